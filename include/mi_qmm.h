@@ -36,9 +36,9 @@
 extern "C" {
 #endif
 
-#define MI_ABI_VERSION 6  /* 2: mi_argmax takes a workspace; 3: mi_gelu_mlp_f32;
+#define MI_ABI_VERSION 7  /* 2: mi_argmax takes a workspace; 3: mi_gelu_mlp_f32;
                              4: mi_argmax_noalloc; 5: the qmm workspace entries;
-                             6: mi_qmm_affine_qkv_norm_rope */
+                             6: mi_qmm_affine_qkv_norm_rope; 7: mi_sdpa_ws */
 
 enum mi_dtype { MI_F32 = 0, MI_F16 = 1, MI_BF16 = 2 };
 
@@ -232,6 +232,20 @@ int mi_qmm_affine_qkv_norm_rope(const void *x, const uint32_t *const w[3],
 int mi_sdpa(const void *q, const void *k, const void *v, void *out, int64_t B, int64_t H,
             int64_t HK, int64_t Lq, int64_t Lk, int64_t D, int64_t kv_cap, float scale,
             int causal, int out_layout, int dtype, void *stream);
+
+/* mi_sdpa with a workspace: a call of few query rows (Lq <= 8) over many keys
+ * (Lk > 1024) then cuts the keys into parts that run as workgroups of their
+ * own, and a second kernel adds them (the same sums in another order: within
+ * rounding of mi_sdpa, deterministic for a shape). workspace: device memory of
+ * mi_sdpa_workspace_bytes(...) bytes (0: no parts at this shape), 16-byte
+ * aligned, no initialization needed; NULL, short or misaligned, or a shape
+ * without parts: mi_sdpa. Calls sharing a workspace must not overlap. */
+int64_t mi_sdpa_workspace_bytes(int64_t B, int64_t H, int64_t HK, int64_t Lq, int64_t Lk,
+                                int64_t D);
+int mi_sdpa_ws(const void *q, const void *k, const void *v, void *out, int64_t B, int64_t H,
+               int64_t HK, int64_t Lq, int64_t Lk, int64_t D, int64_t kv_cap, float scale,
+               int causal, int out_layout, int dtype, void *workspace, int64_t workspace_bytes,
+               void *stream);
 
 /* mlx_lm.models.activations.swiglu(g, u) = silu(g) * u, each op in T:
  * y = T(T(g * T(sigmoid(g))) * u). n elements. */

@@ -24,7 +24,7 @@ import torch
 
 PKG = Path(__file__).resolve().parent.parent
 LIB_PATH = Path(os.environ.get("MI_QMM_LIB", PKG / "libmiqmm.so"))
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 MI_F32, MI_F16, MI_BF16 = 0, 1, 2
 MI_OK, MI_ERR_ARG, MI_ERR_UNSUPPORTED, MI_ERR_LAUNCH = 0, 1, 2, 3
@@ -62,6 +62,9 @@ SIGNATURES: dict[str, list] = {
                                     _I64, _I64, _I, _I, _F, _I, _I, _F, _F, _I64, _I64, _I64,
                                     _I, _P],
     "mi_sdpa": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F, _I, _I, _I, _P],
+    "mi_sdpa_workspace_bytes": [_I64, _I64, _I64, _I64, _I64, _I64],
+    "mi_sdpa_ws": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _I64, _I64, _F, _I, _I, _I, _P,
+                   _I64, _P],
     "mi_swiglu": [_P, _P, _P, _I64, _I, _P],
     "mi_shortconv": [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I, _P],
     "mi_linear_f32": [_P, _P, _P, _P, _I64, _I64, _I64, _I, _P],
@@ -73,7 +76,8 @@ SIGNATURES: dict[str, list] = {
 }
 RESTYPES = {"mi_last_error": ctypes.c_char_p, "mi_argmax_workspace_bytes": ctypes.c_int64,
             "mi_gelu_mlp_f32_workspace_bytes": ctypes.c_int64,
-            "mi_qmm_workspace_bytes": ctypes.c_int64}
+            "mi_qmm_workspace_bytes": ctypes.c_int64,
+            "mi_sdpa_workspace_bytes": ctypes.c_int64}
 
 _lock = threading.Lock()
 _lib = None
@@ -379,6 +383,22 @@ def b_norm_rope(ins, outs, p):
                               _stream(x)), "norm_rope")
 
 
+def sdpa(q, k, v, o, Lk: int, cap: int, scale: float, causal: int, layout: int) -> None:
+    """mi_sdpa over checked tensors, with the split-key workspace where the
+    shape has one."""
+    B, H, Lq, D = q.shape
+    HK, stream = k.shape[1], _stream(q)
+    nbytes = lib().mi_sdpa_workspace_bytes(B, H, HK, Lq, Lk, D) if Lq <= 8 and Lk > 1024 else 0
+    if nbytes:
+        ws = _workspace("sdpa", q.device, stream, nbytes, 4 << 20)
+        _check(lib().mi_sdpa_ws(_ptr(q), _ptr(k), _ptr(v), _ptr(o), B, H, HK, Lq, Lk, D, cap,
+                                scale, causal, layout, _dt(q), _ptr(ws), ws.numel(), stream),
+               "sdpa")
+        return
+    _check(lib().mi_sdpa(_ptr(q), _ptr(k), _ptr(v), _ptr(o), B, H, HK, Lq, Lk, D, cap, scale,
+                         causal, layout, _dt(q), stream), "sdpa")
+
+
 def b_sdpa(ins, outs, p):
     q, k, v = ins
     (o,) = outs
@@ -392,9 +412,7 @@ def b_sdpa(ins, outs, p):
     want = (B, H, Lq, D) if layout == 0 else (B, Lq, H, D)
     if tuple(o.shape) != want or o.dtype != q.dtype or k.dtype != q.dtype or v.dtype != q.dtype:
         raise ValueError(f"sdpa output must be {q.dtype} {want}")
-    _check(lib().mi_sdpa(_ptr(q), _ptr(k), _ptr(v), _ptr(o), B, H, HK, Lq, Lk, D, Lk,
-                         float(p["scale"]), int(p.get("causal", 1)), layout, _dt(q), _stream(q)),
-           "sdpa")
+    sdpa(q, k, v, o, Lk, Lk, float(p["scale"]), int(p.get("causal", 1)), layout)
 
 
 def b_swiglu(ins, outs, p):

@@ -256,9 +256,7 @@ def scaled_dot_product_attention(q, k, v, scale: float, mask: str | None = "caus
     hip._require_gpu(q)
     if tuple(v.shape) != tuple(k.shape) or k.dtype != q.dtype or v.dtype != q.dtype:
         raise ValueError("k and v must match each other and q's dtype")
-    hip._check(hip.lib().mi_sdpa(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), B, H, HK,
-                                 Lq, Lk, D, cap, float(scale), int(mask == "causal"),
-                                 int(out_layout), hip._dt(q), hip._stream(q)), "sdpa")
+    hip.sdpa(q, k, v, o, Lk, cap, float(scale), int(mask == "causal"), int(out_layout))
     return o
 
 

@@ -131,3 +131,15 @@ def test_product_code_never_imports_the_oracle():
         assert not re.search(r"^\s*(import|from)\s+oracle\b", text, flags=re.M), py
     for src in (ROOT / "metal-autotune_amd" / "csrc").glob("*"):
         assert "orc_" not in src.read_text(), src
+
+
+def test_sdpa_workspace_query_needs_no_device(lib):
+    """Split decode calls (Lq <= 8 past 1024 keys): one fp32 state (D sums, a
+    maximum, a row sum) per split and query row; 0 elsewhere."""
+    lib.mi_sdpa_workspace_bytes.restype = ctypes.c_int64
+    lib.mi_sdpa_workspace_bytes.argtypes = [ctypes.c_int64] * 6
+    f = lib.mi_sdpa_workspace_bytes
+    assert f(1, 32, 8, 1, 1024, 128) == 0 and f(1, 32, 8, 9, 4096, 128) == 0
+    assert f(1, 32, 8, 1, 1025, 128) == 9 * 32 * 130 * 4     # 33 tiles: 9 splits of 4
+    assert f(1, 32, 8, 1, 8192, 128) == 64 * 32 * 130 * 4    # 512 workgroups
+    assert f(64, 64, 8, 1, 8192, 64) == 0                    # the heads alone fill the chip
