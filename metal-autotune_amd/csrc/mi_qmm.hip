@@ -32,50 +32,10 @@
 // the q/k RMSNorm, RoPE and the transposed cache write to its sums).
 #include <math.h>
 
-#include "mi_common.h"
+#include "mi_qmm_common.h"
 
 namespace mi {
 namespace {
-
-enum Epi { EPI_STORE = 0, EPI_RESID = 1, EPI_SPLIT3 = 2, EPI_DUAL = 3, EPI_SWIGLU = 4,
-           EPI_GROUP3 = 5, EPI_HEADNR = 6 };
-
-// weight rows each output element combines (EPI_GROUP3 selects one weight per tile)
-constexpr int epi_parts(int e) {
-    return e == EPI_SPLIT3 ? 3 : ((e == EPI_DUAL || e == EPI_SWIGLU) ? 2 : 1);
-}
-
-struct QParams {
-    const void *x;             // T [M, K]
-    const uint32_t *w[3];      // packed weights per part
-    const void *s[3];          // scales per part
-    const void *b[3];          // biases per part
-    int64_t noff[3];           // row offset of each part inside its weight
-    const void *resid;         // T [M, Nout] (EPI_RESID)
-    void *y0;                  // T [M, Nout]
-    void *y1;                  // T [M, Nout] (EPI_SPLIT3, EPI_DUAL)
-    int64_t M, Nout, K;
-    int64_t pn[3];             // EPI_GROUP3: N of each part (Nout = their sum)
-    void *py[3];               // EPI_GROUP3: output of each part, T [M, pn[i]]
-    int gs;
-    int gs_log2;               // log2(gs): group sizes are powers of two
-    int wk;                    // K-split waves (qmm_mfma_kernel)
-    int sbp;                   // qmm_mfma_kernel: groups per row of a wave's scale/bias table
-    int n4;                    // qmm_mfma_mixed_kernel: feature tiles taken as 128-token tiles
-    int sbninst;               // qmm_mfma_kernel: DMA instructions per scale/bias table array
-    unsigned sbmagic;          // ceil(2^20 / (sbp / 2)): v / (sbp / 2) as (v * sbmagic) >> 20
-    int ks;                    // K parts (kpart_count): each is split over the wk waves
-    int kslice;                // k values a scale/bias table covers (a wave chunk, or all of K)
-    int kint;                  // interleaved K split (kint_of): wave w takes stages w, w + wk, ...
-    float *part;               // non-null: write K part blockIdx.z's sums, fp32 [ks, M, Nout]
-    // EPI_HEADNR (the parts are q, k, v; py[] = q_out [B, Hq, L, D], k_cache,
-    // v_cache [B, Hkv, cap, D]; D = 128)
-    const void *nw[2];         // q_norm, k_norm: T [D]
-    int64_t L;                 // tokens per sequence (M = B L)
-    int64_t cap, pos0;         // cache rows per head; first row written
-    int64_t offset;            // RoPE position of a sequence's token 0
-    float eps, log2base, rscale;
-};
 
 // K parts of the MFMA path: a function of (M, K) alone, so every entry point
 // and epilogue (and the tile shape) gives an output element the same sums in
@@ -92,482 +52,8 @@ inline int kpart_count(int64_t M, int64_t K) {
     return (M <= 8 || M > 128 || K < 4096) ? 1 : KPARTS;
 }
 
-template <typename T> __device__ __forceinline__ float swiglu1(float g, float u) {
-    const float gt = (float)cvt<T>(g);
-    const float sig = (float)cvt<T>(1.0f / (1.0f + __expf(-gt)));
-    const float act = (float)cvt<T>(gt * sig);
-    return act * (float)cvt<T>(u);
-}
-
-// The arrays one workgroup reads and writes, held as scalar fields with
-// select accessors: the kernels never modify the QParams argument (a modified
-// copy whose arrays are indexed in loops ends up in scratch memory).
-struct Bound {
-    const uint32_t *w0, *w1, *w2;
-    const void *s0, *s1, *s2;
-    const void *b0, *b1, *b2;
-    int64_t o0, o1, o2;  // row offset of each part inside its weight
-    void *y0;            // this workgroup's output
-    int64_t Nout;        // its width
-    int gp;              // EPI_GROUP3 / EPI_HEADNR: the part it lies in
-    __device__ const uint32_t *w(int i) const { return i == 0 ? w0 : (i == 1 ? w1 : w2); }
-    __device__ const void *s(int i) const { return i == 0 ? s0 : (i == 1 ? s1 : s2); }
-    __device__ const void *b(int i) const { return i == 0 ? b0 : (i == 1 ? b1 : b2); }
-    __device__ int64_t noff(int i) const { return i == 0 ? o0 : (i == 1 ? o1 : o2); }
-};
-
-// Binds a workgroup whose first output feature is nb. EPI_GROUP3: the three
-// weights and outputs are concatenated along N and the host guarantees every
-// part's N is a multiple of each tile width, so the whole tile lies in one
-// part: bind that part as part 0 and make nb relative to it.
-template <int EPI>
-__device__ __forceinline__ Bound bind(const QParams &p, int64_t &nb) {
-    Bound q = {p.w[0], p.w[1], p.w[2], p.s[0], p.s[1], p.s[2], p.b[0], p.b[1], p.b[2],
-               p.noff[0], p.noff[1], p.noff[2], p.y0, p.Nout, 0};
-    if constexpr (EPI == EPI_GROUP3 || EPI == EPI_HEADNR) {
-        const int64_t e0 = p.pn[0], e1 = p.pn[0] + p.pn[1];
-        const bool p0 = nb < e0, p1 = !p0 && nb < e1;
-        nb -= p0 ? 0 : (p1 ? e0 : e1);
-        q.w0 = p0 ? p.w[0] : (p1 ? p.w[1] : p.w[2]);
-        q.s0 = p0 ? p.s[0] : (p1 ? p.s[1] : p.s[2]);
-        q.b0 = p0 ? p.b[0] : (p1 ? p.b[1] : p.b[2]);
-        q.y0 = p0 ? p.py[0] : (p1 ? p.py[1] : p.py[2]);
-        q.Nout = p0 ? p.pn[0] : (p1 ? p.pn[1] : p.pn[2]);
-        q.gp = p0 ? 0 : (p1 ? 1 : 2);
-    }
-    return q;
-}
-
-// Epilogue for one output element (m, n) of the output sub-space.
-template <typename T, int EPI>
-__device__ __forceinline__ void epi1(const QParams &p, const Bound &bd, int64_t m, int64_t n,
-                                     const float *acc) {
-    T *y0 = (T *)bd.y0;
-    const int64_t o = m * bd.Nout + n;
-    if constexpr (EPI == EPI_STORE || EPI == EPI_GROUP3 || EPI == EPI_HEADNR) {
-        y0[o] = cvt<T>(acc[0]);
-    } else if constexpr (EPI == EPI_RESID) {
-        y0[o] = cvt<T>(pin32<T>((float)((const T *)p.resid)[o] + (float)cvt<T>(acc[0])));
-    } else if constexpr (EPI == EPI_SPLIT3) {
-        // split(3): parts 0, 1, 2 are B, C, x; outputs C and T(B * x)
-        y0[o] = cvt<T>(acc[1]);
-        ((T *)p.y1)[o] = cvt<T>((float)cvt<T>(acc[0]) * (float)cvt<T>(acc[2]));
-    } else if constexpr (EPI == EPI_DUAL) {
-        y0[o] = cvt<T>(acc[0]);
-        ((T *)p.y1)[o] = cvt<T>(acc[1]);
-    } else {
-        y0[o] = cvt<T>(swiglu1<T>(acc[0], acc[1]));
-    }
-}
-
-// Whether epi4 takes its vector path at (m, n): in range, four whole features.
-__device__ __forceinline__ bool epi4_vec(const QParams &p, const Bound &bd, int64_t m, int64_t n) {
-    return m < p.M && n + 4 <= bd.Nout && !(bd.Nout & 3);
-}
-
-// EPI_RESID: the residual's four values at (m, n) for epi4's vector path,
-// loaded ahead so a wave's loads are all in flight before its first store
-// (each epi4 loading its own had waited for every load in turn); zeros where
-// the vector path does not run (the element path loads its own).
-template <typename T>
-__device__ __forceinline__ uint2 resid4(const QParams &p, const Bound &bd, int64_t m, int64_t n) {
-    return epi4_vec(p, bd, m, n) ? ld8((const T *)p.resid + m * bd.Nout + n) : make_uint2(0u, 0u);
-}
-
-// Epilogue for 4 consecutive output features n..n+3 of token m; acc[part][e].
-// rpre: EPI_RESID's residual from resid4 (null: loaded here).
-template <typename T, int EPI, int P>
-__device__ __forceinline__ void epi4(const QParams &p, const Bound &bd, int64_t m, int64_t n,
-                                     const float (&acc)[P][4], const uint2 *rpre = nullptr) {
-    if (m >= p.M || n >= bd.Nout) return;
-    if (n + 4 > bd.Nout || (bd.Nout & 3)) {  // ragged tail: element stores
-        for (int e = 0; e < 4 && n + e < bd.Nout; ++e) {
-            float a[P];
-#pragma unroll
-            for (int q = 0; q < P; ++q) a[q] = acc[q][e];
-            epi1<T, EPI>(p, bd, m, n + e, a);
-        }
-        return;
-    }
-    const int64_t o = m * bd.Nout + n;
-    float v[4];
-    if constexpr (EPI == EPI_STORE || EPI == EPI_GROUP3 || EPI == EPI_HEADNR) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[0][e];
-    } else if constexpr (EPI == EPI_RESID) {
-        const uint2 rr = rpre ? *rpre : ld8((const T *)p.resid + o);
-        typedef typename Vec<T>::x4 V4;
-        const V4 rv = __builtin_bit_cast(V4, rr);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = pin32<T>((float)rv[e] + (float)cvt<T>(acc[0][e]));
-    } else if constexpr (EPI == EPI_SPLIT3) {
-        float bx[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = acc[1][e];
-            bx[e] = (float)cvt<T>(acc[0][e]) * (float)cvt<T>(acc[2][e]);
-        }
-        st8((T *)p.y1 + o, pack4<T>(bx));
-    } else if constexpr (EPI == EPI_DUAL) {
-        float u[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            v[e] = acc[0][e];
-            u[e] = acc[1][e];
-        }
-        st8((T *)p.y1 + o, pack4<T>(u));
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = swiglu1<T>(acc[0][e], acc[1][e]);
-    }
-    st8((T *)bd.y0 + o, pack4<T>(v));
-}
-
-// ---------------------------------------------------------------------------
-// GEMV / generic path
-
-template <typename T, int VPC>
-__device__ __forceinline__ void load_x(const T *xp, float (&xf)[VPC]) {
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int i = 0; i < VPC; i += 4) {
-            const uint4 r = ld16(xp + i);
-            xf[i] = __uint_as_float(r.x);
-            xf[i + 1] = __uint_as_float(r.y);
-            xf[i + 2] = __uint_as_float(r.z);
-            xf[i + 3] = __uint_as_float(r.w);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < VPC; i += 8) {
-            float f[8];
-            unpack8<T>(ld16(xp + i), f);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) xf[i + j] = f[j];
-        }
-    }
-}
-
-template <typename T, int BITS, int MR, int EPI>
-__global__ __launch_bounds__(256) void qmv_kernel(QParams p) {
-    constexpr int P = epi_parts(EPI);
-    constexpr int VPW = 32 / BITS;
-    constexpr int VPC = 4 * VPW;
-    const int lane = threadIdx.x & 63;
-    const int j = lane & 15;
-    int64_t nb = (int64_t)blockIdx.x * 16;
-    const Bound bd = bind<EPI>(p, nb);
-    const int64_t n = nb + (threadIdx.x >> 6) * 4 + (lane >> 4);
-    const int64_t m0 = (int64_t)blockIdx.y * MR;
-    const int64_t K = p.K, cpr = K / VPC, G = K >> p.gs_log2;
-    const int mr = (int)((p.M - m0) < MR ? (p.M - m0) : MR);
-    const T *x = (const T *)p.x + m0 * K;
-
-    float acc[P][MR];
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-#pragma unroll
-        for (int m = 0; m < MR; ++m) acc[q][m] = 0.0f;
-
-    // out-of-range rows/tokens read clamped, valid addresses (no branch around
-    // loads); their sums are never stored
-    const int64_t nrow = n < bd.Nout ? n : bd.Nout - 1;
-    const uint32_t *wr[P];
-    const T *sr[P];
-    const T *br[P];
-#pragma unroll
-    for (int q = 0; q < P; ++q) {
-        const int64_t row = bd.noff(q) + nrow;
-        wr[q] = bd.w(q) + row * (K / VPW);
-        sr[q] = (const T *)bd.s(q) + row * G;
-        br[q] = (const T *)bd.b(q) + row * G;
-    }
-#pragma unroll 2
-    for (int64_t c = j; c < cpr; c += 16) {
-        const int64_t k0 = c * VPC;
-        float qf[P][VPC];
-        float sc[P], bi[P];
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-            const uint4 wv = ld16_nt(wr[q] + c * 4);
-            const uint32_t words[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-            for (int i = 0; i < VPC; ++i)
-                qf[q][i] =
-                    (float)((words[i / VPW] >> ((i % VPW) * BITS)) & ((1u << BITS) - 1u));
-            sc[q] = (float)sr[q][k0 >> p.gs_log2];
-            bi[q] = (float)br[q][k0 >> p.gs_log2];
-        }
-#pragma unroll
-        for (int m = 0; m < MR; ++m) {
-            float xf[VPC];
-            load_x<T, VPC>(x + (m < mr ? m : mr - 1) * K + k0, xf);
-            float dx = 0.0f;
-#pragma unroll
-            for (int i = 0; i < VPC; ++i) dx += xf[i];
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                float dq = 0.0f;
-#pragma unroll
-                for (int i = 0; i < VPC; ++i) dq = __builtin_fmaf(xf[i], qf[q][i], dq);
-                acc[q][m] += sc[q] * dq + bi[q] * dx;
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-#pragma unroll
-        for (int m = 0; m < MR; ++m) {
-            acc[q][m] = row16_sum(acc[q][m]);  // the row's 16 lanes
-        }
-    if (j == 0 && n < bd.Nout) {
-#pragma unroll
-        for (int m = 0; m < MR; ++m) {
-            if (m < mr) {
-                float a[P];
-#pragma unroll
-                for (int q = 0; q < P; ++q) a[q] = acc[q][m];
-                epi1<T, EPI>(p, bd, m0 + m, n, a);
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Decode GEMV (M <= 4, 4-bit, bf16/fp16): the nibbles never go through a
-// float conversion. (w >> 4j) & 0x000F000F | MAGIC packs nibbles j and j+4 of a
-// word as the two 16-bit floats MAG + q exactly (bf16: 0x4300 = 128, ulp 1 up
-// to 256; fp16: 0x6400 = 1024, ulp 1), so one v_and_or makes a pair and
-// v_dot2_f32_{bf16,f16} multiplies it with the x pair (x[k], x[k+4]):
-//   sum_k x_k (MAG + q_k) = D  ->  s*sum(x q) + b*sum(x) = s*D + (b - MAG*s)*sum(x).
-// x is staged once per workgroup in LDS already permuted into those pairs,
-// with per-32-value chunk sums. Weight chunks are loaded 8 per lane before use.
-
-template <typename T> struct Magic;
-template <> struct Magic<bf16> {
-    static constexpr uint32_t pair = 0x43004300u;
-    static constexpr float value = 128.0f;
-    static __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
-        typedef __bf16 v2 __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b),
-                                               c, false);
-    }
-};
-template <> struct Magic<f16> {
-    static constexpr uint32_t pair = 0x64006400u;
-    static constexpr float value = 1024.0f;
-    static __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
-        typedef _Float16 v2 __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(v2, a), __builtin_bit_cast(v2, b), c,
-                                      false);
-    }
-};
-
-// ((w >> 4j) & 0x000F000F) | Mg::pair -- the magic pair of nibbles j and
-// j + 4 of w -- in fewer instructions: the even and odd nibbles as bytes
-// (lo, hi) once per word, then one byte permute per pair that interleaves two
-// of those bytes with the magic exponent byte. Same bits.
-template <typename T>
-__device__ __forceinline__ uint32_t magic_pair(uint32_t w, int j) {
-    constexpr uint32_t e = (Magic<T>::pair >> 8) & 0xFFu;  // the exponent byte (0x43 / 0x64)
-    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-    // v_perm_b32 bytes: 0..3 from the second operand, 4..7 from the first
-    const uint32_t sel = (j & 2) ? 0x04030401u : 0x04020400u;
-    return __builtin_amdgcn_perm(e * 0x01010101u, (j & 1) ? hi : lo, sel);
-}
-
-constexpr int QV_BATCH = 8;  // 16-byte weight chunks in flight per lane
-
-inline int64_t qmv_dot2_lds_bytes(int mr, int64_t K) { return mr * K * 2 + mr * (K / 32) * 4; }
-
-// A workgroup of blockDim.x / 64 waves owns 64 / LPR output rows per wave (LPR
-// lanes a row, below): 4 waves, or for single-output epilogues without PF up
-// to 16 (WIDE), sized by the host so the grid spreads the rows evenly over the
-// CUs. Wider workgroups are not used for the others: batches of two or three
-// weight rows take more than the 128 registers a lane may hold in a 16-wave
-// workgroup, and under PF the staging barriers wait for the x loads of every
-// wave, which queue behind the weight stream (one 10-wave workgroup per CU at
-// N = 9728 waited 2.3 us for x against 1.5 us with 4 waves: 6.1 against 5.6
-// us a launch).
-// PF (4 waves at 16 lanes a row; also wide workgroups of a row a wave): the x
-// loads, then the first weight batch, are issued before x is staged, so the
-// weight stream runs under the staging and its two barriers (x first: vmcnt
-// retires in issue order, so waiting for x then leaves the weights in
-// flight). Each thread holds at most two x chunks (K / 8 <= 2 blockDim.x). It
-// costs the batch registers through the staging, which pays when the grid
-// fits the chip in one round and not at N = 151936.
-constexpr bool qmv_dot2_wide_ok(int epi) { return epi_parts(epi) == 1 && epi != EPI_GROUP3; }
-
-// LPR: lanes per output row, 16 (4 rows a wave) or 64 (a row a wave, for long
-// K: a K = 9728 row is 19 chunks a lane at 16 lanes, loaded in three batches
-// one after another, and about 5 at 64, one batch).
-template <typename T, int MR, int EPI, bool PF = false, bool WIDE = false, int LPR = 16>
-__global__ __launch_bounds__(WIDE ? 1024 : 256) void qmv_dot2_kernel(QParams p) {
-    static_assert(!WIDE || qmv_dot2_wide_ok(EPI), "wide workgroups: single output");
-    static_assert(LPR == 16 || (LPR == 64 && qmv_dot2_wide_ok(EPI)), "a row a wave: single output");
-    static_assert(!PF || MR == 1, "PF: one token");
-    static_assert(!PF || !WIDE || LPR == 64, "PF in wide workgroups: a row a wave");
-    constexpr int RPW = 64 / LPR;  // rows a wave
-    constexpr int P = epi_parts(EPI);
-    typedef Magic<T> Mg;
-    extern __shared__ uint4 xs_pairs[];  // [MR][K/8] pair blocks, then [MR][K/32] sums
-    const int64_t K = p.K, words = K / 8, cpr = K / 32, G = K >> p.gs_log2;
-    float *xsum = (float *)(xs_pairs + MR * words);
-    const int lane = threadIdx.x & 63, j = lane & (LPR - 1);
-    const int bs = WIDE ? (int)blockDim.x : 256;  // threads
-    int64_t nb = (int64_t)blockIdx.x * ((bs >> 6) * RPW);
-    const Bound bd = bind<EPI>(p, nb);
-    const int64_t n = nb + (threadIdx.x >> 6) * RPW + lane / LPR;
-    const int64_t nrow = n < bd.Nout ? n : bd.Nout - 1;
-    const int64_t m0 = (int64_t)blockIdx.y * MR;
-    const int mr = (int)((p.M - m0) < MR ? (p.M - m0) : MR);
-
-    const uint32_t *wr[P];
-    const T *sr[P];
-    const T *br[P];
-#pragma unroll
-    for (int q = 0; q < P; ++q) {
-        const int64_t row = bd.noff(q) + nrow;
-        wr[q] = bd.w(q) + row * (K / 8);
-        sr[q] = (const T *)bd.s(q) + row * G;
-        br[q] = (const T *)bd.b(q) + row * G;
-    }
-
-    uint4 wv[P][QV_BATCH];
-    T sv[P][QV_BATCH], bv[P][QV_BATCH];
-    auto load_batch = [&](int64_t base) {
-#pragma unroll
-        for (int i = 0; i < QV_BATCH; ++i) {
-            const int64_t c = base + LPR * i;
-            const int64_t cc = c < cpr ? c : cpr - 1;
-            const int64_t g = (cc * 32) >> p.gs_log2;
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                wv[q][i] = ld16_nt(wr[q] + 4 * cc);
-                sv[q][i] = sr[q][g];
-                bv[q][i] = br[q][g];
-            }
-        }
-    };
-
-    // stage x rows as pairs (e[i], e[i+4]) of each 8-value block
-    const T *x = (const T *)p.x + m0 * K;
-    auto pairs = [](const uint4 d) {
-        return make_uint4(__builtin_amdgcn_perm(d.z, d.x, 0x05040100u),
-                          __builtin_amdgcn_perm(d.z, d.x, 0x07060302u),
-                          __builtin_amdgcn_perm(d.w, d.y, 0x05040100u),
-                          __builtin_amdgcn_perm(d.w, d.y, 0x07060302u));
-    };
-    const int nw = (int)words;  // 32-bit index math: MR * K < 2^31
-    if constexpr (PF) {
-        // Every thread issues both loads (a clamped, valid chunk when past the
-        // end) so the issue order, and with it the waits, is the same in all
-        // waves: x, then the weights (K / 8 <= 2 bs)
-        uint4 d[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            int idx = (int)threadIdx.x + bs * t;
-            idx = idx < MR * nw ? idx : MR * nw - 1;
-            const int m = MR == 1 ? 0 : idx / nw, w = idx - m * nw;
-            d[t] = ld16(x + (int64_t)(m < mr ? m : mr - 1) * K + 8 * w);
-        }
-        __builtin_amdgcn_sched_barrier(0);  // keep the x loads ahead of the weights'
-        load_batch(j);
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int64_t idx = threadIdx.x + bs * t;
-            if (idx < MR * words) xs_pairs[idx] = pairs(d[t]);
-        }
-    } else {
-        for (int idx = threadIdx.x; idx < MR * nw; idx += bs) {
-            const int m = MR == 1 ? 0 : idx / nw, w = idx - m * nw;
-            xs_pairs[idx] = pairs(ld16(x + (int64_t)(m < mr ? m : mr - 1) * K + 8 * w));
-        }
-    }
-    __syncthreads();
-    const int ncpr = (int)cpr;
-    for (int idx = threadIdx.x; idx < MR * ncpr; idx += bs) {
-        const int m = MR == 1 ? 0 : idx / ncpr, c = idx - m * ncpr;
-        float s = 0.0f;
-#pragma unroll
-        for (int wi = 0; wi < 4; ++wi) {
-            const uint4 v = xs_pairs[m * words + 4 * c + wi];
-            float f[8];
-            unpack8<T>(v, f);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s += f[i];
-        }
-        xsum[idx] = s;
-    }
-    __syncthreads();
-
-    float acc[P][MR];
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-#pragma unroll
-        for (int m = 0; m < MR; ++m) acc[q][m] = 0.0f;
-
-    for (int64_t base = j; base < cpr; base += LPR * QV_BATCH) {
-        // (Without PF the compiler sinks each chunk's loads to its use behind
-        // the `c >= cpr` exit, so a lane fetches its chunks one after another;
-        // at 58 registers eight waves per SIMD keep the loads in flight.)
-        if (!PF || base != j) load_batch(base);
-#pragma unroll
-        for (int i = 0; i < QV_BATCH; ++i) {
-            const int64_t c = base + LPR * i;
-            if (c >= cpr) break;
-#pragma unroll
-            for (int q = 0; q < P; ++q) {
-                const uint32_t wd[4] = {wv[q][i].x, wv[q][i].y, wv[q][i].z, wv[q][i].w};
-                uint32_t qp[4][4];
-#pragma unroll
-                for (int wi = 0; wi < 4; ++wi)
-#pragma unroll
-                    for (int jj = 0; jj < 4; ++jj)
-                        qp[wi][jj] = magic_pair<T>(wd[wi], jj);
-                const float s = (float)sv[q][i];
-                const float bb = __builtin_fmaf(-Mg::value, s, (float)bv[q][i]);
-#pragma unroll
-                for (int m = 0; m < MR; ++m) {
-                    float d = 0.0f;
-#pragma unroll
-                    for (int wi = 0; wi < 4; ++wi) {
-                        const uint4 xp = xs_pairs[m * words + 4 * c + wi];
-                        d = Mg::dot2(qp[wi][0], xp.x, d);
-                        d = Mg::dot2(qp[wi][1], xp.y, d);
-                        d = Mg::dot2(qp[wi][2], xp.z, d);
-                        d = Mg::dot2(qp[wi][3], xp.w, d);
-                    }
-                    acc[q][m] += s * d + bb * xsum[m * cpr + c];
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-#pragma unroll
-        for (int m = 0; m < MR; ++m) {
-            acc[q][m] = row16_sum(acc[q][m]);  // the row's 16 lanes
-            if constexpr (LPR == 64) {  // then the wave's four 16-lane sums
-                const int v = __builtin_bit_cast(int, acc[q][m]);
-                const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(v, 0));
-                const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(v, 16));
-                const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(v, 32));
-                const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(v, 48));
-                acc[q][m] = (r0 + r1) + (r2 + r3);
-            }
-        }
-    if (j == 0 && n < bd.Nout) {
-#pragma unroll
-        for (int m = 0; m < MR; ++m) {
-            if (m < mr) {
-                float a[P];
-#pragma unroll
-                for (int q = 0; q < P; ++q) a[q] = acc[q][m];
-                epi1<T, EPI>(p, bd, m0 + m, n, a);
-            }
-        }
-    }
+template <typename T> constexpr int dtype_of() {
+    return sizeof(T) == 4 ? MI_F32 : (__is_same(T, bf16) ? MI_BF16 : MI_F16);
 }
 
 // ---------------------------------------------------------------------------
@@ -608,7 +94,6 @@ template <> struct Mfma<f16> {
 // are a per-lane 32-bit offset plus a scalar stage offset (no VALU address
 // arithmetic in the loop).
 constexpr int XK = 64;  // k values per x stage (128 bytes of a token row)
-constexpr int LDS_PER_CU = 160 * 1024;
 
 template <typename T, int BITS, int A, int C, int WK>
 struct MfmaShape {
@@ -666,14 +151,6 @@ __host__ __device__ inline SbtLayout sbt_layout(int64_t kslice, int gs) {
     return {need, ninst, ninst * 256};
 }
 
-// A raw buffer resource over [base, base + bytes): 32-bit offsets, and reads
-// past the end return zero instead of touching memory.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void *base, uint32_t bytes) {
-    // dword 3: 32-bit data format (gfx9 raw buffer access)
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes,
-                                             0x00020000);
-}
-
 // One stage slot per wave. Measured on MI355X at the Qwen3 prefill shapes
 // (M = 128), it beats rings of two to eight slots: the small footprint lets
 // three workgroups share a CU (three waves per SIMD, which overlap one wave's
@@ -682,18 +159,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void *base, 
 // o_proj 12.1 -> 11.5, bit for bit the same results. (A balanced grid of one
 // workgroup per CU gains nothing from deeper rings either: 25.9 us with one
 // slot, 27.7 us with two or three, dual at N = 8192.)
-
-// s_waitcnt with vmcnt = N and no wait on the other counters (gfx9 encoding:
-// vmcnt[3:0] at bits 3:0 and vmcnt[5:4] at bits 15:14, expcnt 7, lgkmcnt 15).
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit count");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// s_waitcnt lgkmcnt(0) with no wait on vmcnt (63) or expcnt (7)
-__device__ __forceinline__ void wait_lgkmcnt0() {
-    __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));
-}
 
 // Waves per SIMD the register allocation must allow: the single slot exists
 // so three workgroups of four waves share a CU (at most 168 registers a
@@ -1611,22 +1076,6 @@ __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu<A, 4>()))) void qmm_mfma_mi
 // ---------------------------------------------------------------------------
 // dispatch
 
-constexpr int QMV_MR = 8;     // rows per GEMV block (and the GEMV/MFMA switch)
-
-template <typename T, int BITS, int EPI>
-int launch_qmv(const QParams &p, hipStream_t st) {
-    const dim3 grid((unsigned)ceil_div(p.Nout, 16), (unsigned)ceil_div(p.M, QMV_MR));
-    if (p.M == 1)
-        qmv_kernel<T, BITS, 1, EPI><<<grid, 256, 0, st>>>(p);
-    else if (p.M <= 2)
-        qmv_kernel<T, BITS, 2, EPI><<<grid, 256, 0, st>>>(p);
-    else if (p.M <= 4)
-        qmv_kernel<T, BITS, 4, EPI><<<grid, 256, 0, st>>>(p);
-    else
-        qmv_kernel<T, BITS, QMV_MR, EPI><<<grid, 256, 0, st>>>(p);
-    return launch_status("quantized matmul (qmv)");
-}
-
 // k values of the longest of the ks * wk wave chunks of K
 inline int kslice_of(int64_t K, int ks, int wk) {
     return (int)ceil_div(K / XK, (int64_t)ks * wk) * XK;
@@ -1711,21 +1160,6 @@ int launch_mfma_cfg(QParams p, int wk, hipStream_t st) {
     return launch_status("quantized matmul (mfma)");
 }
 
-// Compute units of the current device (cached per device).
-int device_cus() {
-    static int cache[64];
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (cache[dev] == 0) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            n <= 0)
-            n = 256;
-        cache[dev] = n;
-    }
-    return cache[dev];
-}
-
 // qmm_mfma_mixed_kernel over nt feature tiles, the first nb of them as
 // CB * 32-token tiles (four K-split waves).
 template <typename T, int BITS, int A, int EPI, int CB>
@@ -1775,7 +1209,7 @@ int launch_mfma(const QParams &p, hipStream_t st) {
     if (p.ks > 1) {
         if (mfma_lds_bytes<T, BITS, P, 1>(p, wk) <= LDS_PER_CU)
             return launch_mfma_cfg<T, BITS, P, 1, EPI, KM_LOOP>(p, wk, st);
-        return launch_qmv<T, BITS, EPI>(p, st);
+        return gemv_launch(p, EPI, BITS, dtype_of<T>(), st);
     }
     const int64_t nt = ceil_div(p.Nout, 32);
     const bool large = p.M >= 512 || nt * ceil_div(p.M, 64) > 2048;
@@ -1842,80 +1276,7 @@ int launch_mfma(const QParams &p, hipStream_t st) {
     }
     if (mfma_lds_bytes<T, BITS, P, 1>(p, wk) <= LDS_PER_CU)
         return launch_mfma_cfg<T, BITS, P, 1, EPI>(p, wk, st);
-    return launch_qmv<T, BITS, EPI>(p, st);
-}
-
-template <typename T, int EPI>
-int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
-    // weights requested under the x staging when the 4-wave grid is at most
-    // four workgroups per CU (measured: N = 9728 gains, N = 151936 loses),
-    // for single-output epilogues: holding two or three weight rows' batches
-    // through the staging takes 226-256 registers, one or two waves a SIMD
-    // (the gate/up dual at M = 1, N = 9728: 10.9 us with PF, 8.6 without)
-    const int64_t gy = ceil_div(p.M, mr);
-    const bool pf = epi_parts(EPI) == 1 && mr == 1 && ceil_div(p.Nout, 16) * gy <= 1024 &&
-                    p.K / 8 <= 512;
-    // A row a wave (LPR 64) for single-output launches over long rows (K >
-    // 4096, more than 8 chunks a lane at 16 lanes a row). Waves per workgroup
-    // without PF: as many as spread the rows evenly over the CUs in one round
-    // of workgroups (N = 9728 at 4 rows a wave: 10 waves, 244 workgroups, at
-    // most 40 rows a CU, where 16-row workgroups put 48 on some CUs and 32 on
-    // the others: M = 2 7.5 -> 7.2 us, M = 4 11.0 -> 9.6); 4 when the rows
-    // take more than one round of 16-wave workgroups, for the grouped q/k/v
-    // epilogue, whose workgroups each lie inside one part, and for the
-    // several-output ones.
-    constexpr bool wide_ok = qmv_dot2_wide_ok(EPI);
-    const bool row_wave = wide_ok && !pf && p.K / 32 > 128;
-    const int rpw = row_wave ? 1 : 4;
-    int waves = 4;
-    if constexpr (wide_ok) {
-        const int64_t wv = ceil_div(p.Nout, rpw * (int64_t)device_cus());
-        if (!pf && wv <= 16) waves = wv < 4 ? 4 : (int)wv;
-    }
-    const int bs = 64 * waves;
-    const dim3 grid((unsigned)ceil_div(p.Nout, rpw * waves), (unsigned)gy);
-    const size_t lds = (size_t)qmv_dot2_lds_bytes(mr, p.K);
-    if (pf) {
-        qmv_dot2_kernel<T, 1, EPI, true><<<grid, bs, lds, st>>>(p);
-    } else if (!row_wave && waves == 4) {
-        if (mr == 1)
-            qmv_dot2_kernel<T, 1, EPI><<<grid, bs, lds, st>>>(p);
-        else if (mr == 2)
-            qmv_dot2_kernel<T, 2, EPI><<<grid, bs, lds, st>>>(p);
-        else
-            qmv_dot2_kernel<T, 4, EPI><<<grid, bs, lds, st>>>(p);
-    } else if constexpr (wide_ok) {
-        // a row a wave takes PF too at M = 1 while x fits two chunks a thread
-        // (Qwen3's down_proj at decode, 10-wave workgroups: 6.7 -> 5.6 us)
-        if (row_wave && mr == 1 && p.K / 8 <= 2 * bs) {
-            if (waves == 4)
-                qmv_dot2_kernel<T, 1, EPI, true, false, 64><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 1, EPI, true, true, 64><<<grid, bs, lds, st>>>(p);
-        } else if (row_wave && waves == 4) {
-            if (mr == 1)
-                qmv_dot2_kernel<T, 1, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
-            else if (mr == 2)
-                qmv_dot2_kernel<T, 2, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 4, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
-        } else if (row_wave) {
-            if (mr == 1)
-                qmv_dot2_kernel<T, 1, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
-            else if (mr == 2)
-                qmv_dot2_kernel<T, 2, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 4, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
-        } else {
-            if (mr == 1)
-                qmv_dot2_kernel<T, 1, EPI, false, true><<<grid, bs, lds, st>>>(p);
-            else if (mr == 2)
-                qmv_dot2_kernel<T, 2, EPI, false, true><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 4, EPI, false, true><<<grid, bs, lds, st>>>(p);
-        }
-    }
-    return launch_status("quantized matmul (dot2 qmv)");
+    return gemv_launch(p, EPI, BITS, dtype_of<T>(), st);
 }
 
 // Shapes the MFMA kernel takes (16-bit T): it addresses x and each weight
@@ -1930,9 +1291,6 @@ template <typename T, int EPI>
 int launch_typed(const QParams &p, int bits, hipStream_t st) {
     const bool mfma = (sizeof(T) == 2) && mfma_shape_ok(p.M, p.K, p.noff[2] + p.Nout, p.gs, bits);
     if constexpr (sizeof(T) == 2) {
-        const int mr = p.M == 1 ? 1 : (p.M == 2 ? 2 : 4);
-        if (bits == 4 && p.M <= 4 && qmv_dot2_lds_bytes(mr, p.K) <= 65536)
-            return launch_qmv_dot2<T, EPI>(p, mr, st);
         if (mfma) {
             QParams q = p;
             q.ks = kpart_count(p.M, p.K);
@@ -1940,7 +1298,7 @@ int launch_typed(const QParams &p, int bits, hipStream_t st) {
             return bits == 4 ? launch_mfma<T, 4, EPI>(q, st) : launch_mfma<T, 8, EPI>(q, st);
         }
     }
-    return bits == 4 ? launch_qmv<T, 4, EPI>(p, st) : launch_qmv<T, 8, EPI>(p, st);
+    return gemv_launch(p, EPI, bits, dtype_of<T>(), st);
 }
 
 // The K-part launch (p.part set): 128-token tiles when M > 64, so a part

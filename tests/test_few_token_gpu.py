@@ -1,0 +1,89 @@
+"""The few-token quantized matmul (2 to 8 rows) at the edges of its shapes.
+
+Bars: the region criterion max|c - r| <= 1e-2 max|r| against the factored
+float oracle (the same per-group sums), and the fused epilogues bit for bit
+against their op streams (one K split and group order per (M, K)).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+from conftest import packed_to_torch, rng, to_np, to_torch
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+from autotuner_runtime import ops  # noqa: E402
+
+
+def _dev(seed, N, K, gs, bits, dtype):
+    wq, s, b = oracle.quantize_affine(rng(seed).normal(0, 0.02, (N, K)).astype(np.float32), gs, bits,
+                                      dtype)
+    return (wq, s, b), (packed_to_torch(wq), to_torch(s, dtype), to_torch(b, dtype))
+
+
+def _close(got, want):
+    err = np.abs(to_np(got).astype(np.float64) - want).max() / np.abs(want).max()
+    assert err <= 1e-2, err
+
+
+@pytest.mark.parametrize("M,N,K,gs,bits,dtype", [
+    (3, 16, 32, 32, 4, "bfloat16"),       # one group: seven waves without work
+    (5, 40, 96, 32, 4, "float16"),        # an odd group count (single groups), a ragged last tile
+    (8, 200, 320, 64, 4, "bfloat16"),     # 5 groups
+    (6, 72, 640, 64, 4, "float16"),       # 10 groups in pairs, runs of one and none
+    (4, 64, 1152, 128, 4, "bfloat16"),    # 9 groups of four steps
+    (7, 88, 4160, 64, 4, "bfloat16"),     # 16 waves, an odd group count
+    (2, 56, 160, 32, 8, "bfloat16"),      # 8 bits, odd count
+    (8, 200, 512, 32, 8, "float16"),      # 8 bits in pairs
+    (5, 24, 1088, 64, 8, "float16"),
+    (3, 104, 896, 128, 8, "bfloat16"),
+    (1, 96, 8192, 64, 8, "bfloat16"),     # one token, long rows
+    (8, 48, 9728, 64, 4, "bfloat16"),     # x past the LDS: two blocks of four rows
+    (5, 32, 20480, 64, 8, "float16"),     # ... of three and two
+    (2, 48, 90112, 128, 8, "bfloat16"),   # not one row fits: the generic kernel
+])
+def test_few_token_shapes(M, N, K, gs, bits, dtype):
+    r = rng(5000 + M + N + K)
+    x = oracle.round_to(r.normal(0, 1, (1, M, K)), dtype)
+    res = oracle.round_to(r.normal(0, 1, (1, M, N)), dtype)
+    host, w = _dev(5001 + N, N, K, gs, bits, dtype)
+    host2, w2 = _dev(5002 + N, N, K, gs, bits, dtype)
+    xd, rd = to_torch(x, dtype), to_torch(res, dtype)
+    y = ops.quantized_matmul(xd, *w, group_size=gs, bits=bits)
+    _close(y, oracle.qmm_factored(x, *host, gs, bits, dtype))
+    assert torch.equal(ops.qmm_residual(xd, *w, rd, gs, bits), rd + y)
+    u = ops.quantized_matmul(xd, *w2, group_size=gs, bits=bits)
+    y1, u1 = ops.qmm_dual(xd, *w, *w2, gs, bits)
+    assert torch.equal(y1, y) and torch.equal(u1, u)
+    assert torch.equal(ops.qmm_dual(xd, *w, *w2, gs, bits, swiglu=True), ops.swiglu(y, u))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("D", [64, 104])
+def test_few_token_split_and_grouped(bits, D):
+    """split(3) parts that start on and off a 16-feature tile, and q/k/v in one
+    launch, against the plain projection."""
+    M, K = 5, 1024
+    r = rng(5100 + D)
+    xd = to_torch(oracle.round_to(r.normal(0, 1, (1, M, K)), "bfloat16"), "bfloat16")
+    _, w = _dev(5101, 3 * D, K, 64, bits, "bfloat16")
+    t = ops.quantized_matmul(xd, *w, bits=bits)
+    c, bx = ops.qmm_split_gate(xd, *w, bits=bits)
+    assert torch.equal(c, t[..., D:2 * D]) and torch.equal(bx, t[..., :D] * t[..., 2 * D:])
+    parts = [_dev(5102 + i, n, K, 64, bits, "bfloat16")[1] for i, n in enumerate((96, 32, 64))]
+    for got, p in zip(ops.qmm_grouped3(xd, parts, bits=bits), parts):
+        assert torch.equal(got, ops.quantized_matmul(xd, *p, bits=bits))
+
+
+def test_few_token_unaligned_scales():
+    """Scales and biases that are views off a 16-byte boundary (the kernel's DMA
+    cannot take them) run the generic kernel."""
+    M, N, K = 4, 33, 320
+    x = oracle.round_to(rng(5200).normal(0, 1, (M, K)), "bfloat16")
+    host, w = _dev(5201, N, K, 64, 4, "bfloat16")
+    y = ops.quantized_matmul(to_torch(x, "bfloat16"), *(t[1:] for t in w))
+    _close(y, oracle.qmm_factored(x, *(a[1:] for a in host), 64, 4, "bfloat16"))
