@@ -149,14 +149,20 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float *__restrict
 
 // Config 1's whole MLP in one launch: y = gelu(x W1^T + b1) W2^T + b2, fp32.
 // Workgroup (c, rb) takes hidden units [64 c, 64 c + 64) for token rows
-// [8 rb, 8 rb + 8): phase 1 computes those gelu(h) values into LDS (each a
-// sequential fma chain over k, plus b1); phase 2 multiplies them into a
-// partial y tile [8, N] over its 64 hidden units and stores it in the
-// workspace. The last workgroup of a row block to finish (a ticket counter
-// per row block) adds the partials of chunks 0, 1, 2, ... in that fixed order,
-// then b2, and writes y, so the result does not depend on which workgroup
-// finished last. It then resets the counter: the workspace's counters are zero
-// before the first call and after every call.
+// [8 rb, 8 rb + 8): phase 1 computes those gelu(h) values into LDS, phase 2
+// multiplies them into a partial y tile [8, N] over its 64 hidden units and
+// stores it in the workspace. In both, four lanes share a weight row and take
+// every fourth 16 bytes of it (64-byte pieces, each lane's loads independent;
+// their fma chains meet in a quad sum): with a row a lane, every step of the
+// chain waited for a load of 64 rows' 16 bytes. The last workgroup of a row
+// block to finish (a ticket counter per row block) adds the partials of chunks
+// 0, 1, 2, ... in that fixed order, then b2, and writes y, so the result does not
+// depend on which workgroup finished last. It then resets the counter: the
+// workspace's counters are zero before the first call and after every call.
+// The partials are stored with agent scope (written through) and acknowledged
+// before the ticket, where a release fence writes back the whole XCD's L2.
+// Bound: the chain of launch, W1, W2 (requested under phase 1), ticket and the
+// partials' round trips: 32 x 256 -> 1024 -> 256 54 -> 19 us, 512 rows 196 -> 51.
 constexpr int MLP_HT = 64;      // hidden units per workgroup
 constexpr int MLP_RT = 8;       // token rows per workgroup
 constexpr int MLP_THREADS = 256;
@@ -166,99 +172,174 @@ __device__ __forceinline__ float gelu_erf(float v) {
     return v * (1.0f + erff(v / 1.41421356237f)) / 2.0f;
 }
 
+// The sum over a lane's quad, the same bits in its four lanes.
+__device__ __forceinline__ float quad_sum(float v) {
+    v += dpp_f32<0xB1>(v);  // lane ^ 1
+    v += dpp_f32<0x4E>(v);  // lane ^ 2
+    return v;
+}
+
+// a[r] += w . x[r] over four consecutive k, for the MLP_RT rows at x (row pitch
+// in floats).
+__device__ __forceinline__ void mlp_fma(float (&a)[MLP_RT], const float4 w, const float *x,
+                                        int pitch) {
+#pragma unroll
+    for (int r = 0; r < MLP_RT; ++r) {
+        const float4 v = *(const float4 *)(x + r * pitch);
+        a[r] = __builtin_fmaf(v.x, w.x, a[r]);
+        a[r] = __builtin_fmaf(v.y, w.y, a[r]);
+        a[r] = __builtin_fmaf(v.z, w.z, a[r]);
+        a[r] = __builtin_fmaf(v.w, w.w, a[r]);
+    }
+}
+
+// y = the sum of the C partial planes, in order, plus the bias: V values a load
+// of the block's rows x N.
+template <int V>
+__device__ __forceinline__ void mlp_reduce(const float *part, const float *__restrict__ b2,
+                                           float *__restrict__ y, int rows, int64_t N,
+                                           int64_t plane, int C, int t) {
+    typedef float VF __attribute__((ext_vector_type(V)));
+    constexpr int FLY = 16;
+    for (int64_t i = (int64_t)t * V; i < rows * N; i += MLP_THREADS * V) {
+        VF s;
+        for (int c0 = 0; c0 < C; c0 += FLY) {
+            VF v[FLY];
+#pragma unroll
+            for (int j = 0; j < FLY; ++j)
+                v[j] = *(const VF *)(part + (c0 + j < C ? c0 + j : C - 1) * plane + i);
+#pragma unroll
+            for (int j = 0; j < FLY; ++j)
+                if (c0 + j < C) s = c0 + j == 0 ? v[j] : s + v[j];
+        }
+        const int64_t n = i % N;
+#pragma unroll
+        for (int e = 0; e < V; ++e) y[i + e] = s[e] + (b2 ? b2[n + e] : 0.0f);
+    }
+}
+
 __global__ __launch_bounds__(MLP_THREADS) void gelu_mlp_f32_kernel(
     const float *__restrict__ x, const float *__restrict__ w1, const float *__restrict__ b1,
     const float *__restrict__ w2, const float *__restrict__ b2, float *__restrict__ y,
-    float *__restrict__ part, unsigned *__restrict__ tickets, int64_t M, int64_t K, int64_t H,
-    int64_t N) {
+    float *part, unsigned *__restrict__ tickets, int64_t M, int64_t K, int64_t H, int64_t N) {
     extern __shared__ __attribute__((aligned(16))) float mlp_lds[];
     float *xs = mlp_lds;                       // [MLP_RT][K]
     float *hs = mlp_lds + MLP_RT * K;          // [MLP_RT][MLP_HT]
     __shared__ int last;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, quad = t >> 2, ql = t & 3;
     const int64_t c = blockIdx.x, rb = blockIdx.y;
     const int64_t C = gridDim.x;
     const int64_t r0 = rb * MLP_RT;
     const int rows = (int)(M - r0 < MLP_RT ? M - r0 : MLP_RT);
+    const int64_t hbase = c * MLP_HT;
+    const int hn4 = (int)(H - hbase < MLP_HT ? H - hbase : MLP_HT) / 4;
+    const int k4 = (int)(K / 4);
+
+    // W1: the quad's row, BATCH of the lane's chunks in flight (chunks past the
+    // row read its last one; their products are skipped)
+    constexpr int BATCH = 16;
+    const int64_t hj = hbase + quad, hrow = hj < H ? hj : H - 1;
+    const float4 *wr1 = (const float4 *)(w1 + hrow * K);
+    float4 wv[BATCH];
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) wv[i] = wr1[ql + 4 * i < k4 ? ql + 4 * i : k4 - 1];
+    // W2: the first NB output columns' chunks, requested under phase 1
+    constexpr int NB = 4, HQ = MLP_HT / 16;
+    float4 w2v[NB][HQ];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        const int64_t n = quad + 64 * i, nc = n < N ? n : N - 1;
+        const float4 *wr = (const float4 *)(w2 + nc * H + hbase);
+#pragma unroll
+        for (int j = 0; j < HQ; ++j) w2v[i][j] = wr[ql + 4 * j < hn4 ? ql + 4 * j : hn4 - 1];
+    }
+    const float bias1 = b1 ? b1[hrow] : 0.0f;
 
     // stage the row block of x (rows past M read as zero)
-    for (int64_t i = t; i < MLP_RT * K / 4; i += MLP_THREADS) {
-        const int64_t r = (4 * i) / K, k = 4 * i - r * K;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (r < rows) v = *(const float4 *)(x + (r0 + r) * K + k);
-        *(float4 *)(xs + r * K + k) = v;
-    }
-    __syncthreads();
-
-    // phase 1: lane j of wave w computes hidden unit 64 c + j for rows w, w + 4
-    {
-        const int j = t & 63, w = t >> 6;
-        const int64_t hj = c * MLP_HT + j;
-        const int64_t hrow = hj < H ? hj : H - 1;  // clamped, valid row
-        const float *wr = w1 + hrow * K;
-        float a0 = 0.0f, a1 = 0.0f;
-        for (int64_t k = 0; k < K; k += 4) {
-            const float4 wv = *(const float4 *)(wr + k);
-            const float4 xa = *(const float4 *)(xs + w * K + k);
-            const float4 xb = *(const float4 *)(xs + (w + 4) * K + k);
-            a0 = __builtin_fmaf(xa.x, wv.x, a0);
-            a0 = __builtin_fmaf(xa.y, wv.y, a0);
-            a0 = __builtin_fmaf(xa.z, wv.z, a0);
-            a0 = __builtin_fmaf(xa.w, wv.w, a0);
-            a1 = __builtin_fmaf(xb.x, wv.x, a1);
-            a1 = __builtin_fmaf(xb.y, wv.y, a1);
-            a1 = __builtin_fmaf(xb.z, wv.z, a1);
-            a1 = __builtin_fmaf(xb.w, wv.w, a1);
+    for (int r = 0; r < MLP_RT; ++r)
+        for (int i = t; i < k4; i += MLP_THREADS) {
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (r < rows) v = ((const float4 *)(x + (r0 + r) * K))[i];
+            ((float4 *)(xs + r * K))[i] = v;
         }
-        const float bias = b1 ? b1[hrow] : 0.0f;
-        hs[w * MLP_HT + j] = hj < H ? gelu_erf(a0 + bias) : 0.0f;
-        hs[(w + 4) * MLP_HT + j] = hj < H ? gelu_erf(a1 + bias) : 0.0f;
+    __syncthreads();
+
+    // phase 1: hidden unit 64 c + quad for every row
+    {
+        float a[MLP_RT];
+#pragma unroll
+        for (int r = 0; r < MLP_RT; ++r) a[r] = 0.0f;
+        for (int i0 = ql; i0 < k4; i0 += 4 * BATCH) {
+            if (i0 != ql) {
+#pragma unroll
+                for (int i = 0; i < BATCH; ++i) wv[i] = wr1[i0 + 4 * i < k4 ? i0 + 4 * i : k4 - 1];
+            }
+#pragma unroll
+            for (int i = 0; i < BATCH; ++i)
+                if (i0 + 4 * i < k4) mlp_fma(a, wv[i], xs + 4 * (i0 + 4 * i), (int)K);
+        }
+#pragma unroll
+        for (int r = 0; r < MLP_RT; ++r) a[r] = quad_sum(a[r]);
+        // lane ql finishes rows 2 ql and 2 ql + 1
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const float v = ql == 0 ? a[e] : (ql == 1 ? a[2 + e] : (ql == 2 ? a[4 + e] : a[6 + e]));
+            hs[(2 * ql + e) * MLP_HT + quad] = hj < H ? gelu_erf(v + bias1) : 0.0f;
+        }
     }
     __syncthreads();
 
-    // phase 2: thread t takes output columns n = t, t + 256, ... for all rows
-    const int64_t hbase = c * MLP_HT;
-    const int hn = (int)(H - hbase < MLP_HT ? H - hbase : MLP_HT);  // a multiple of 4
+    // phase 2: output columns quad, quad + 64, ... for all rows
     float *pc = part + c * (M * N);
-    for (int64_t n = t; n < N; n += MLP_THREADS) {
-        const float *wr = w2 + n * H + hbase;
-        float acc[MLP_RT];
+    for (int64_t n0 = quad; n0 < N; n0 += 64 * NB) {
+        if (n0 != quad) {
 #pragma unroll
-        for (int r = 0; r < MLP_RT; ++r) acc[r] = 0.0f;
-        for (int hh = 0; hh < hn; hh += 4) {
-            const float4 wv = *(const float4 *)(wr + hh);
+            for (int i = 0; i < NB; ++i) {
+                const int64_t n = n0 + 64 * i, nc = n < N ? n : N - 1;
+                const float4 *wr = (const float4 *)(w2 + nc * H + hbase);
 #pragma unroll
-            for (int r = 0; r < MLP_RT; ++r) {
-                const float4 hv = *(const float4 *)(hs + r * MLP_HT + hh);
-                acc[r] = __builtin_fmaf(hv.x, wv.x, acc[r]);
-                acc[r] = __builtin_fmaf(hv.y, wv.y, acc[r]);
-                acc[r] = __builtin_fmaf(hv.z, wv.z, acc[r]);
-                acc[r] = __builtin_fmaf(hv.w, wv.w, acc[r]);
+                for (int j = 0; j < HQ; ++j) w2v[i][j] = wr[ql + 4 * j < hn4 ? ql + 4 * j : hn4 - 1];
             }
         }
 #pragma unroll
-        for (int r = 0; r < MLP_RT; ++r)
-            if (r < rows) pc[(r0 + r) * N + n] = acc[r];
+        for (int i = 0; i < NB; ++i) {
+            const int64_t n = n0 + 64 * i;
+            if (n >= N) break;  // (the quad's four lanes alike)
+            float a[MLP_RT];
+#pragma unroll
+            for (int r = 0; r < MLP_RT; ++r) a[r] = 0.0f;
+#pragma unroll
+            for (int j = 0; j < HQ; ++j)
+                if (ql + 4 * j < hn4) mlp_fma(a, w2v[i][j], hs + 4 * (ql + 4 * j), MLP_HT);
+#pragma unroll
+            for (int r = 0; r < MLP_RT; ++r) a[r] = quad_sum(a[r]);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int r = 2 * ql + e;
+                const float v = ql == 0 ? a[e] : (ql == 1 ? a[2 + e] : (ql == 2 ? a[4 + e] : a[6 + e]));
+                if (r < rows)
+                    __hip_atomic_store(pc + (r0 + r) * N + n, v, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
     }
 
     // phase 3: the last workgroup of this row block reduces the partials
-    __threadfence();  // release: this workgroup's partials before its ticket
-    __syncthreads();
+    __builtin_amdgcn_s_waitcnt(0);  // this wave's partials are at the agent's level ...
+    __syncthreads();                // ... and every wave's, before the ticket
     if (t == 0) {
-        const unsigned ticket = atomicAdd(&tickets[rb], 1u);
+        const unsigned ticket =
+            __hip_atomic_fetch_add(&tickets[rb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         last = ticket == (unsigned)(C - 1);
     }
     __syncthreads();
     if (!last) return;
-    __threadfence();  // acquire: every partial of the row block is visible
-    for (int64_t i = t; i < (int64_t)rows * N; i += MLP_THREADS) {
-        const int64_t r = i / N, n = i - r * N;
-        const int64_t o = (r0 + r) * N + n;
-        float s = part[o];
-        for (int64_t cc = 1; cc < C; ++cc) s += part[cc * (M * N) + o];
-        if (b2) s += b2[n];
-        y[o] = s;
-    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // no stale copy of a partial is read
+    // (16 bytes a load where the rows allow: 16 partials in flight a thread)
+    if (N % 4 == 0)
+        mlp_reduce<4>(part + r0 * N, b2, y + r0 * N, rows, N, M * N, (int)C, t);
+    else
+        mlp_reduce<1>(part + r0 * N, b2, y + r0 * N, rows, N, M * N, (int)C, t);
     if (t == 0) __hip_atomic_store(&tickets[rb], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
