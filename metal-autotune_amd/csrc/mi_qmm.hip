@@ -1185,16 +1185,29 @@ int launch_mfma_mixed3(QParams p, int nb, int cus, hipStream_t st) {
     return launch_status("quantized matmul (mfma, three tile sizes)");
 }
 
-// Tile choice (measured on MI355X over the Qwen3 prefill shapes, M = 128): one
+// Past 128 tokens a launch's time follows the workgroups of its fullest CU:
+// first + more (n - 1) for n = ceil(workgroups / CUs), whatever N, K and bits
+// (the time scale, a function of K, is common to the tiles). Fitted, in 0.1 us
+// at K = 2560, to N 1024 / 2048 / 2560 / 6144 by K 2048 to 9728 and the duals
+// N 8192 and 9728 at 129, 200, 256, 320, 384 and 501 tokens, 4 and 8 bits
+// (features x tokens): 32x32 58 + 37, 32x64 71 + 51, 32x128 98 + 88, 64x64
+// 94 + 82, 64x128 134 + 125. Before, 32x64 below 512 tokens or 32x32 past a
+// K of about 9000, 64x128 from 512, and two thresholds on the width between.
+// 4 bits, 501 tokens: 6144 x 2560 33.6 -> 26.7 us, 2560 x 4096 24.7 -> 19.7,
+// 2560 x 9728 63.8 -> 40.3, 2048 x 8192 44.7 -> 26.5; dual 9728 x 2560 at 384
+// 60 -> 52; a Qwen3 layer's 501-token chunk 236 -> 201 us.
+inline int64_t round_cost(const QParams &p, int tn, int C, int first, int more) {
+    const int64_t wgs = ceil_div(p.Nout, 32 * tn) * ceil_div(p.M, 32 * C);
+    return first + more * (ceil_div(wgs, device_cus()) - 1);
+}
+
+// Tile choice. Up to M = 128 (measured over the Qwen3 prefill shapes): one
 // 32-feature tile per part (A = P) and 64-token tiles (C = 2) -- the smallest
 // tiles that still reuse each x fragment across two MFMA columns -- give the
 // most workgroups for these narrow-N GEMMs; 32-token tiles when 64-token tiles
-// would leave fewer than 128 workgroups (half the CUs). From M = 512 (or past
-// 2048 workgroups) 128-token tiles, two 32-feature tiles per wave for
-// single-part outputs: re-reading x per narrow tile then costs more than the
-// lost parallelism (LFM2 at M = 2048: down_proj 198 -> 99 us, out_proj 42 ->
-// 30 us, the gate/up dual 257 -> 234 us). Tiles never change the numerics:
-// the K split (wk) and each output's accumulation order are fixed by K.
+// would leave fewer than 128 workgroups (half the CUs). Past 128 tokens the
+// tile comes from round_cost. Tiles never change the numerics: the K split
+// (wk) and each output's accumulation order are fixed by (M, K).
 // K must split into wk slices of whole 64-value x stages. A tile whose rings
 // and scale/bias tables (which grow with K) exceed the LDS steps down to the
 // next smaller one, and past the smallest the GEMV kernel runs instead.
@@ -1212,29 +1225,55 @@ int launch_mfma(const QParams &p, hipStream_t st) {
         return gemv_launch(p, EPI, BITS, dtype_of<T>(), st);
     }
     const int64_t nt = ceil_div(p.Nout, 32);
-    const bool large = p.M >= 512 || nt * ceil_div(p.M, 64) > 2048;
-    if constexpr (P == 1) {
-        // (both widths. 8-bit took 32x128 tiles while its 64x128 tile
-        // spilled; without the spill, LFM2's 8-bit out/down_proj at M = 2048
-        // went 84.9 -> 64.4 us on average. The grouped q/k/v epilogue binds
-        // one part per tile, so it takes 64-feature tiles only when every
-        // part is a multiple of 64: LFM2's q/k/v at M = 2048, 6.35 -> 6.30 ms
-        // a prefill against 32-feature tiles)
-        const bool al2 = EPI != EPI_GROUP3 ||
-                         (p.pn[0] % 64 == 0 && p.pn[1] % 64 == 0 && p.pn[2] % 64 == 0);
-        // wide single-part 4-bit outputs take 64x128 tiles from M = 128
-        // (N = 9728: 23.1 -> 21.3 us; narrower N loses parallelism)
-        const bool wide = EPI != EPI_GROUP3 && p.M >= 128 && nt >= 256;
-        if ((large || wide) && al2 && mfma_lds_bytes<T, BITS, 2, 4>(p, wk) <= LDS_PER_CU)
-            return launch_mfma_cfg<T, BITS, 2, 4, EPI>(p, wk, st);
-        if constexpr (EPI == EPI_GROUP3) {
-            if (large && mfma_lds_bytes<T, BITS, 1, 4>(p, wk) <= LDS_PER_CU)
-                return launch_mfma_cfg<T, BITS, 1, 4, EPI>(p, wk, st);
+    // (the grouped q/k/v epilogue binds one part per tile, so it takes
+    // 64-feature tiles only when every part is a multiple of 64)
+    const bool al2 = EPI != EPI_GROUP3 ||
+                     (p.pn[0] % 64 == 0 && p.pn[1] % 64 == 0 && p.pn[2] % 64 == 0);
+    if constexpr (P <= 2) {
+        if (p.M > 128) {
+            enum { NONE, T11, T12, T14, T22, T24 } best = NONE;
+            int64_t cost = 0;
+            auto offer = [&](decltype(best) tile, int64_t lds, int tn, int C, int first, int more) {
+                const int64_t c = round_cost(p, tn, C, first, more);
+                if (lds > LDS_PER_CU || (best != NONE && c >= cost)) return;
+                best = tile;
+                cost = c;
+            };
+            if constexpr (P == 1) {
+                offer(T11, mfma_lds_bytes<T, BITS, 1, 1>(p, wk), 1, 1, 58, 37);
+                offer(T12, mfma_lds_bytes<T, BITS, 1, 2>(p, wk), 1, 2, 71, 51);
+                if constexpr (EPI == EPI_GROUP3) {
+                    if (!al2) offer(T14, mfma_lds_bytes<T, BITS, 1, 4>(p, wk), 1, 4, 98, 88);
+                }
+            }
+            if (al2 && (P == 1 || nt * ceil_div(p.M, 64) >= 128)) {
+                offer(T22, mfma_lds_bytes<T, BITS, 2, 2>(p, wk), 3 - P, 2, 94, 82);
+                offer(T24, mfma_lds_bytes<T, BITS, 2, 4>(p, wk), 3 - P, 4, 134, 125);
+            }
+            if constexpr (P == 1) {
+                if (best == T11) return launch_mfma_cfg<T, BITS, 1, 1, EPI>(p, wk, st);
+                if (best == T12) return launch_mfma_cfg<T, BITS, 1, 2, EPI>(p, wk, st);
+                if constexpr (EPI == EPI_GROUP3) {
+                    if (best == T14) return launch_mfma_cfg<T, BITS, 1, 4, EPI>(p, wk, st);
+                }
+            }
+            if (best == T22) return launch_mfma_cfg<T, BITS, 2, 2, EPI>(p, wk, st);
+            if (best == T24) return launch_mfma_cfg<T, BITS, 2, 4, EPI>(p, wk, st);
         }
     }
-    if constexpr (P == 2) {
-        if (large && mfma_lds_bytes<T, BITS, 2, 4>(p, wk) <= LDS_PER_CU)
+    // Very wide outputs up to 128 tokens: re-reading x per narrow tile costs
+    // more than the lost parallelism. Single-part outputs of 8192 features or
+    // more take 64x128 tiles at M = 128 (N = 9728: 23.1 -> 21.3 us; narrower N
+    // loses parallelism).
+    const bool large = nt * ceil_div(p.M, 64) > 2048;
+    const bool wide = P == 1 && EPI != EPI_GROUP3 && p.M >= 128 && nt >= 256;
+    if constexpr (P <= 2) {
+        if ((large || wide) && al2 && mfma_lds_bytes<T, BITS, 2, 4>(p, wk) <= LDS_PER_CU)
             return launch_mfma_cfg<T, BITS, 2, 4, EPI>(p, wk, st);
+    }
+    if constexpr (EPI == EPI_GROUP3) {
+        if (large && mfma_lds_bytes<T, BITS, 1, 4>(p, wk) <= LDS_PER_CU)
+            return launch_mfma_cfg<T, BITS, 1, 4, EPI>(p, wk, st);
     }
     // 64 < M <= 128 whose 64-token grid (2 nt workgroups) puts one workgroup
     // more on some CUs than on others: mixed tiles make it exactly two per CU,
