@@ -15,6 +15,7 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
+import functools
 import os
 import threading
 from pathlib import Path
@@ -135,7 +136,9 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # the handle torch.cuda.current_stream(t.device) wraps, without making the
+    # Stream object (1 us a call, once or twice in every launch)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _dt(t: torch.Tensor) -> int:
@@ -157,8 +160,9 @@ def _quant(w: torch.Tensor, s: torch.Tensor, b: torch.Tensor, bits: int, gs: int
         raise ValueError(f"packed weights must be a 2-d uint32 array, got {w.dtype} {tuple(w.shape)}")
     if bits not in (4, 8):
         raise ValueError(f"bits={bits}; this build covers 4 and 8")
-    N, K = w.shape[0], w.shape[1] * 32 // bits
-    if gs <= 0 or K % gs or tuple(s.shape) != (N, K // gs) or tuple(b.shape) != (N, K // gs):
+    N, words = w.shape
+    K = words * 32 // bits
+    if gs <= 0 or K % gs or not s.shape == b.shape == (N, K // gs):
         raise ValueError(f"scales {tuple(s.shape)} / biases {tuple(b.shape)} do not match "
                          f"w {tuple(w.shape)} at {bits} bits, group {gs}")
     if s.dtype != b.dtype:
@@ -216,14 +220,20 @@ def _qmm_dims(x, w, s, b, p):
 
 
 def _out_like(y, x, N, name="output"):
-    if y.dtype != x.dtype or tuple(y.shape) != (*x.shape[:-1], N):
+    if y.dtype != x.dtype or y.shape != (*x.shape[:-1], N):
         raise ValueError(f"{name} must be {x.dtype} {(*x.shape[:-1], N)}, got {y.dtype} {tuple(y.shape)}")
+
+
+@functools.lru_cache(maxsize=1024)
+def _qmm_workspace_bytes(M, N, K, gs, bits, dt) -> int:
+    """mi_qmm_workspace_bytes, a function of these numbers alone."""
+    return int(lib().mi_qmm_workspace_bytes(M, N, K, gs, bits, dt))
 
 
 def _qmm_workspace(x, M, N, K, gs, bits, dt):
     """The K-part workspace of the _ws entries at this shape, or None (one
     K part: the plain entry)."""
-    nbytes = int(lib().mi_qmm_workspace_bytes(M, N, K, gs, bits, dt))
+    nbytes = _qmm_workspace_bytes(M, N, K, gs, bits, dt)
     if nbytes == 0:
         return None
     return _workspace("qmm", x.device, _stream(x), nbytes, 8 << 20)

@@ -240,7 +240,8 @@ class LoadedKernel:
         signature. ``checked_elsewhere``: a size-generic caller that serves
         only sizes this kernel was checked at; recorded signatures then do not
         restrict the call (the fallback predicate still does)."""
-        key = (checked_elsewhere,) + tuple((tuple(a.shape), a.dtype) for a in inputs)
+        # (a torch.Size hashes and compares as the tuple it is)
+        key = (checked_elsewhere, *[a.shape for a in inputs], *[a.dtype for a in inputs])
         hit = self._launches.get(key)
         if hit is not None:
             self._launches.move_to_end(key)
@@ -254,11 +255,11 @@ class LoadedKernel:
     def fallback_fires(self, inputs: list[torch.Tensor]) -> bool:
         return self.launch(inputs).fallback
 
-    def _allocate(self, launch: Launch, device, init_value):
+    def _allocate(self, launch: Launch, like: torch.Tensor, init_value):
         if init_value is None:
-            return [torch.empty(s, dtype=d, device=device)
+            return [like.new_empty(s, dtype=d)
                     for s, d in zip(launch.output_shapes, self._out_dtypes)]
-        return [torch.full(s, init_value, dtype=d, device=device)
+        return [torch.full(s, init_value, dtype=d, device=like.device)
                 for s, d in zip(launch.output_shapes, self._out_dtypes)]
 
     def __call__(self, inputs: list[torch.Tensor], init_value: float | None = None,
@@ -276,7 +277,7 @@ class LoadedKernel:
             for kernel, pos in self._stages:
                 table += kernel([table[j] for j in pos], init_value=init_value)
             return [table[j] for j in self._stage_outputs]
-        outputs = self._allocate(launch, inputs[0].device, init_value)
+        outputs = self._allocate(launch, inputs[0], init_value)
         self._entry(inputs, outputs, dict(launch.template))
         return outputs
 

@@ -19,7 +19,7 @@ from . import hip
 
 
 def _empty(shape, like: torch.Tensor, dtype=None) -> torch.Tensor:
-    return torch.empty(shape, dtype=dtype or like.dtype, device=like.device)
+    return like.new_empty(shape, dtype=dtype)
 
 
 def _qp(group_size: int, bits: int) -> dict:
