@@ -193,29 +193,58 @@ __device__ __forceinline__ void mlp_fma(float (&a)[MLP_RT], const float4 w, cons
     }
 }
 
-// y = the sum of the C partial planes, in order, plus the bias: V values a load
-// of the block's rows x N.
+// y = the sum of the C partial planes, in order, plus the bias, over the block's
+// rows x N: U pieces of V values a thread at a time, FLY planes of each
+// requested together (a piece past the end re-reads the thread's first).
+template <int V, int U, int FLY>
+__device__ __forceinline__ void mlp_reduce_by(const float *part, const float *__restrict__ b2,
+                                              float *__restrict__ y, int64_t total, int64_t N,
+                                              int64_t plane, int C, int t) {
+    typedef float VF __attribute__((ext_vector_type(V)));
+    constexpr int STEP = MLP_THREADS * V;
+    for (int64_t i = (int64_t)t * V; i < total; i += STEP * U) {
+        VF s[U];
+        for (int c0 = 0; c0 < C; c0 += FLY) {
+            VF v[FLY][U];
+#pragma unroll
+            for (int j = 0; j < FLY; ++j)
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    v[j][u] = *(const VF *)(part + (c0 + j < C ? c0 + j : C - 1) * plane +
+                                            (i + u * STEP < total ? i + u * STEP : i));
+#pragma unroll
+            for (int j = 0; j < FLY; ++j)
+                if (c0 + j < C)
+#pragma unroll
+                    for (int u = 0; u < U; ++u) s[u] = c0 + j == 0 ? v[j][u] : s[u] + v[j][u];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t o = i + u * STEP;
+            if (o >= total) break;
+            const int64_t n = o % N;
+#pragma unroll
+            for (int e = 0; e < V; ++e) y[o + e] = s[u][e] + (b2 ? b2[n + e] : 0.0f);
+        }
+    }
+}
+
+// A round trip to the partials costs some 2 us, so a thread asks for several
+// pieces at once, and for no more planes than there are: one piece of 16 planes
+// a trip made a row block of 8 x 500 in two planes sixteen trips of 16 loads.
+// 32 rows, 64 -> 128 -> 501 30.4 -> 24.4 us, 1020 -> 2044 -> 509 59 -> 49; 512
+// rows of the latter 252 -> 207, 64 -> 128 -> 501 34 -> 28.
 template <int V>
 __device__ __forceinline__ void mlp_reduce(const float *part, const float *__restrict__ b2,
                                            float *__restrict__ y, int rows, int64_t N,
                                            int64_t plane, int C, int t) {
-    typedef float VF __attribute__((ext_vector_type(V)));
-    constexpr int FLY = 16;
-    for (int64_t i = (int64_t)t * V; i < rows * N; i += MLP_THREADS * V) {
-        VF s;
-        for (int c0 = 0; c0 < C; c0 += FLY) {
-            VF v[FLY];
-#pragma unroll
-            for (int j = 0; j < FLY; ++j)
-                v[j] = *(const VF *)(part + (c0 + j < C ? c0 + j : C - 1) * plane + i);
-#pragma unroll
-            for (int j = 0; j < FLY; ++j)
-                if (c0 + j < C) s = c0 + j == 0 ? v[j] : s + v[j];
-        }
-        const int64_t n = i % N;
-#pragma unroll
-        for (int e = 0; e < V; ++e) y[i + e] = s[e] + (b2 ? b2[n + e] : 0.0f);
-    }
+    const int64_t total = (int64_t)rows * N;
+    if (C <= 4)
+        mlp_reduce_by<V, 16 / V, 4>(part, b2, y, total, N, plane, C, t);
+    else if (C <= 8)
+        mlp_reduce_by<V, V == 4 ? 4 : 8, 8>(part, b2, y, total, N, plane, C, t);
+    else
+        mlp_reduce_by<V, V == 4 ? 2 : 4, 16>(part, b2, y, total, N, plane, C, t);
 }
 
 __global__ __launch_bounds__(MLP_THREADS) void gelu_mlp_f32_kernel(
@@ -242,7 +271,8 @@ __global__ __launch_bounds__(MLP_THREADS) void gelu_mlp_f32_kernel(
     const float4 *wr1 = (const float4 *)(w1 + hrow * K);
     float4 wv[BATCH];
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) wv[i] = wr1[ql + 4 * i < k4 ? ql + 4 * i : k4 - 1];
+    for (int i = 0; i < BATCH; ++i)
+        if (i == 0 || 4 * i < k4) wv[i] = wr1[ql + 4 * i < k4 ? ql + 4 * i : k4 - 1];
     // W2: the first NB output columns' chunks, requested under phase 1
     constexpr int NB = 4, HQ = MLP_HT / 16;
     float4 w2v[NB][HQ];
