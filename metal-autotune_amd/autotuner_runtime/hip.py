@@ -467,22 +467,29 @@ def b_linear_f32(ins, outs, p):
                                int(p.get("act", MI_ACT_NONE)), _stream(x)), "linear_f32")
 
 
-# Workspaces (the K-part sums of the _ws qmm entries, mi_gelu_mlp_f32's
-# tickets and partial sums), zero-filled when made; mi_gelu_mlp_f32 leaves its
-# tickets zero after every call.
+# Workspaces: scratch of the entries that make several launches or sum across
+# workgroups (the K-part sums of the _ws qmm entries, the split decode's partial
+# states, mi_gelu_mlp_f32's tickets and partial sums). Only the tickets need a
+# zero fill when made (mi_gelu_mlp_f32 leaves them zero after every call).
 #
-# Eager calls share one workspace per (kind, device, stream): calls on one
-# stream run in order. A call under HIP graph capture bakes the workspace's
-# address into the graph, and graphs may later replay on different streams at
-# the same time, so a captured call never takes an eager stream's workspace:
-# inside graph_workspaces() every graph captured in the scope shares the
-# scope's own workspaces (its calls are stream-ordered), and a capture outside
-# such a scope gives each call a workspace of its own. Either way the buffer is
-# kept alive as long as the process, since a graph may replay at any time; a
-# workspace that has to grow is replaced and the old one kept alive too.
-_workspaces: dict[tuple, torch.Tensor] = {}
+# Eager calls share one workspace per (thread, kind, device, stream): one
+# thread's calls on one stream run in order, where a second thread may launch
+# between the two launches of a call. A workspace that has to grow at least
+# doubles; the old one goes back to torch's allocator, which hands memory of a
+# stream to later work of that stream.
+#
+# A call under HIP graph capture bakes the workspace's address into the graph,
+# and graphs may later replay on different streams at the same time, so a
+# captured call never takes an eager workspace: inside graph_workspaces() the
+# calls of every graph captured in the scope share the scope's own, one per
+# stream, and a capture outside such a scope gives each call a workspace of its
+# own. Either way the buffer is kept alive as long as the process, since a graph
+# may replay at any time, also one that has to grow (the earlier calls' nodes
+# hold its address). It is made at the size asked for, and a fill, where one is
+# needed, is a node that every replay repeats.
+_captured: dict[tuple, torch.Tensor] = {}
 _retired: list[torch.Tensor] = []
-_scope = threading.local()
+_scope = threading.local()   # .token: the capture scope; .eager: the thread's workspaces
 
 
 @contextlib.contextmanager
@@ -497,23 +504,30 @@ def graph_workspaces():
         _scope.token = prev
 
 
-def _workspace(kind: str, device, stream: int, nbytes: int, minimum: int = 4096) -> torch.Tensor:
-    size = max(nbytes, minimum)
+def _workspace(kind: str, device, stream: int, nbytes: int, minimum: int = 4096,
+               zero: bool = False) -> torch.Tensor:
+    make = torch.zeros if zero else torch.empty
     if torch.cuda.is_current_stream_capturing():
         token = getattr(_scope, "token", None)
-        if token is None:  # a capture of its own: a workspace per call
-            ws = torch.zeros(size, dtype=torch.uint8, device=device)
-            _retired.append(ws)
-            return ws
-        key = (kind, device, token)
-    else:
-        key = (kind, device, stream)
-    ws = _workspaces.get(key)
+        key = (kind, device, stream, token)
+        ws = None if token is None else _captured.get(key)
+        if ws is None or ws.numel() < nbytes:
+            if ws is not None:
+                _retired.append(ws)
+            ws = make(max(nbytes, 4096), dtype=torch.uint8, device=device)
+            if token is None:
+                _retired.append(ws)
+            else:
+                _captured[key] = ws
+        return ws
+    eager = getattr(_scope, "eager", None)
+    if eager is None:
+        eager = _scope.eager = {}
+    key = (kind, device, stream)
+    ws = eager.get(key)
     if ws is None or ws.numel() < nbytes:
-        if ws is not None:
-            _retired.append(ws)
-        ws = torch.zeros(size, dtype=torch.uint8, device=device)
-        _workspaces[key] = ws
+        size = max(nbytes, minimum, 0 if ws is None else 2 * ws.numel())
+        eager[key] = ws = make(size, dtype=torch.uint8, device=device)
     return ws
 
 
@@ -534,7 +548,7 @@ def b_gelu_mlp_f32(ins, outs, p):
         raise ValueError("gelu_mlp_f32 shapes")
     stream = _stream(x)
     nbytes = int(lib().mi_gelu_mlp_f32_workspace_bytes(M, K, H, N))
-    ws = _workspace("gelu_mlp", x.device, stream, nbytes)
+    ws = _workspace("gelu_mlp", x.device, stream, nbytes, zero=True)
     _check(lib().mi_gelu_mlp_f32(_ptr(x), _ptr(w1), _ptr(b1), _ptr(w2), _ptr(b2), _ptr(y), M, K,
                                  H, N, _ptr(ws), ws.numel(), stream), "gelu_mlp_f32")
 
