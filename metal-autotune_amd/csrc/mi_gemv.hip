@@ -33,6 +33,14 @@ __device__ __forceinline__ void load_x(const T *xp, float (&xf)[VPC]) {
     }
 }
 
+// a b + c d with the rounding written out: left to contraction, the compiler
+// fused one product or the other by the epilogue it compiled, and an epilogue's
+// fp32 sums differed from the plain projection's in their last bit.
+__device__ __forceinline__ float fma_mul(float a, float b, float c, float d) {
+#pragma clang fp contract(off)
+    return __builtin_fmaf(a, b, c * d);
+}
+
 template <typename T, int BITS, int MR, int EPI>
 __global__ __launch_bounds__(256) void qmv_kernel(QParams p) {
     constexpr int P = epi_parts(EPI);
@@ -95,7 +103,7 @@ __global__ __launch_bounds__(256) void qmv_kernel(QParams p) {
                 float dq = 0.0f;
 #pragma unroll
                 for (int i = 0; i < VPC; ++i) dq = __builtin_fmaf(xf[i], qf[q][i], dq);
-                acc[q][m] += sc[q] * dq + bi[q] * dx;
+                acc[q][m] += fma_mul(bi[q], dx, sc[q], dq);
             }
         }
     }
@@ -323,7 +331,7 @@ __global__ __launch_bounds__(WIDE ? 1024 : 256) void qmv_dot2_kernel(QParams p) 
                         d = Mg::dot2(qp[wi][2], xp.z, d);
                         d = Mg::dot2(qp[wi][3], xp.w, d);
                     }
-                    acc[q][m] += s * d + bb * xsum[m * cpr + c];
+                    acc[q][m] += fma_mul(s, d, bb, xsum[m * cpr + c]);
                 }
             }
         }

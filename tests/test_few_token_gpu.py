@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 from autotuner_runtime import ops  # noqa: E402
+from workloads.quantize import random_quantized  # noqa: E402
 
 
 def _dev(seed, N, K, gs, bits, dtype):
@@ -87,3 +88,20 @@ def test_few_token_unaligned_scales():
     host, w = _dev(5201, N, K, 64, 4, "bfloat16")
     y = ops.quantized_matmul(to_torch(x, "bfloat16"), *(t[1:] for t in w))
     _close(y, oracle.qmm_factored(x, *(a[1:] for a in host), 64, 4, "bfloat16"))
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M", [1, 3, 8])
+def test_generic_kernel_epilogues_agree(M, bits):
+    """The fp32 kernel's sums are its outputs: an epilogue that rounds a group's
+    sum in another way shows in the last bit."""
+    N, K = 96, 1024
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + bits)
+    xd = torch.randn((1, M, K), generator=gen, device="cuda")
+    w, w2 = (random_quantized(N, K, gen, "cuda", 64, bits, torch.float32) for _ in range(2))
+    t, u = (ops.quantized_matmul(xd, *a, bits=bits) for a in (w, w2))
+    y1, u1 = ops.qmm_dual(xd, *w, *w2, 64, bits)
+    assert torch.equal(y1, t) and torch.equal(u1, u)
+    c, bx = ops.qmm_split_gate(xd, *w, 64, bits)
+    assert torch.equal(c, t[..., 32:64]) and torch.equal(bx, t[..., :32] * t[..., 64:])
