@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void qmv_kernel(QParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Decode GEMV (M <= 4, 4-bit, bf16/fp16): the nibbles never go through a
+// Decode GEMV (M <= 2, 4-bit, bf16/fp16): the nibbles never go through a
 // float conversion. (w >> 4j) & 0x000F000F | MAGIC packs nibbles j and j+4 of a
 // word as the two 16-bit floats MAG + q exactly (bf16: 0x4300 = 128, ulp 1 up
 // to 256; fp16: 0x6400 = 1024, ulp 1), so one v_and_or makes a pair and
@@ -499,7 +499,8 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
     char *sbl = qlds + rows * L.pitch;  // [part][scale, bias][16][G]
 
     // x rows, then the scale and bias rows, 16 bytes a lane; the instructions
-    // are dealt to the waves
+    // are dealt to the waves. Scale and bias rows off a 16-byte boundary, or
+    // whose last tile ends off one, come a value a thread.
     {
         const __amdgpu_buffer_rsrc_t xr =
             buffer_rsrc((const T *)p.x + m0 * K, (uint32_t)(rows * K * (int64_t)sizeof(T)));
@@ -516,11 +517,17 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
         }
         const int chunks = 2 * G, ips = (chunks + 63) >> 6;
         const int64_t left = (bd.Nout - nb) * G * 2;  // the part's rows from nb on
+        const uint32_t bytes = (uint32_t)(left < L.sb ? left : L.sb);
 #pragma unroll
         for (int a = 0; a < 2 * P; ++a) {
             const T *base = (const T *)((a & 1) ? bd.b(a >> 1) : bd.s(a >> 1)) + (bd.noff(a >> 1) + nb) * G;
-            const __amdgpu_buffer_rsrc_t sr =
-                buffer_rsrc(base, (uint32_t)(left < L.sb ? left : L.sb));
+            if ((((uintptr_t)base | bytes) & 15) != 0) {  // (workgroup-uniform)
+                T *dst = (T *)(sbl + a * L.sb);
+                for (int i = threadIdx.x; i < (int)(bytes / sizeof(T)); i += 64 * nw) dst[i] = base[i];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // before the barrier below
+                continue;
+            }
+            const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(base, bytes);
             for (int j = wave; j < ips; j += nw) {
                 const int c = 64 * j + lane;
                 if (c < chunks)
@@ -719,7 +726,7 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
     // without PF: as many as spread the rows evenly over the CUs in one round
     // of workgroups (N = 9728 at 4 rows a wave: 10 waves, 244 workgroups, at
     // most 40 rows a CU, where 16-row workgroups put 48 on some CUs and 32 on
-    // the others: M = 2 7.5 -> 7.2 us, M = 4 11.0 -> 9.6); 4 when the rows
+    // the others: M = 2 7.5 -> 7.2 us); 4 when the rows
     // take more than one round of 16-wave workgroups, for the grouped q/k/v
     // epilogue, whose workgroups each lie inside one part, and for the
     // several-output ones.
@@ -739,10 +746,8 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
     } else if (!row_wave && waves == 4) {
         if (mr == 1)
             qmv_dot2_kernel<T, 1, EPI><<<grid, bs, lds, st>>>(p);
-        else if (mr == 2)
-            qmv_dot2_kernel<T, 2, EPI><<<grid, bs, lds, st>>>(p);
         else
-            qmv_dot2_kernel<T, 4, EPI><<<grid, bs, lds, st>>>(p);
+            qmv_dot2_kernel<T, 2, EPI><<<grid, bs, lds, st>>>(p);
     } else if constexpr (wide_ok) {
         // a row a wave takes PF too at M = 1 while x fits two chunks a thread
         // (Qwen3's down_proj at decode, 10-wave workgroups: 6.7 -> 5.6 us)
@@ -754,44 +759,36 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
         } else if (row_wave && waves == 4) {
             if (mr == 1)
                 qmv_dot2_kernel<T, 1, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
-            else if (mr == 2)
-                qmv_dot2_kernel<T, 2, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
             else
-                qmv_dot2_kernel<T, 4, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
+                qmv_dot2_kernel<T, 2, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
         } else if (row_wave) {
             if (mr == 1)
                 qmv_dot2_kernel<T, 1, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
-            else if (mr == 2)
-                qmv_dot2_kernel<T, 2, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
             else
-                qmv_dot2_kernel<T, 4, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
+                qmv_dot2_kernel<T, 2, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
         } else {
             if (mr == 1)
                 qmv_dot2_kernel<T, 1, EPI, false, true><<<grid, bs, lds, st>>>(p);
-            else if (mr == 2)
-                qmv_dot2_kernel<T, 2, EPI, false, true><<<grid, bs, lds, st>>>(p);
             else
-                qmv_dot2_kernel<T, 4, EPI, false, true><<<grid, bs, lds, st>>>(p);
+                qmv_dot2_kernel<T, 2, EPI, false, true><<<grid, bs, lds, st>>>(p);
         }
     }
     return launch_status("quantized matmul (dot2 qmv)");
 }
 
-// Token rows per workgroup (all of them, halved while x does not fit the LDS),
-// or 0 where qms_kernel does not apply: its DMA takes scale and bias arrays
-// 16-byte aligned and whole 16-byte chunks long, 32-bit offsets, and at least one
-// x row in LDS.
-inline int qms_rows(const QParams &p, int epi) {
-    const int parts = epi_parts(epi), waves = qms_waves(p.K);
-    const int64_t G = p.K >> p.gs_log2;
-    if (p.M > QMV_MR || p.K >= ((int64_t)1 << 24)) return 0;
-    for (int i = 0; i < 3; ++i) {
-        const int64_t rows = epi == EPI_GROUP3 ? p.pn[i] : p.Nout;
-        if (!aligned(p.s[i], 16) || !aligned(p.b[i], 16) || (p.noff[i] * G) % 8 || (rows * G) % 8)
-            return 0;
-    }
+// Whether qms_kernel takes a call's (M, K, group size): up to 8 tokens, 32-bit
+// offsets, and one x row in the LDS beside the scales and biases of three parts,
+// whatever the epilogue has, so that every epilogue of one shape takes it (and
+// adds in its order) or none does.
+inline bool qms_takes(int64_t M, int64_t K, int gs_log2) {
+    return M <= QMV_MR && K < ((int64_t)1 << 24) &&
+           qms_lds(1, K, K >> gs_log2, 3, qms_waves(K)).total <= LDS_PER_CU;
+}
+// Token rows per workgroup: all of them, halved while x does not fit the LDS.
+inline int qms_rows(const QParams &p, int parts) {
     int mr = (int)p.M;
-    while (mr > 0 && qms_lds(mr, p.K, G, parts, waves).total > LDS_PER_CU) mr = mr > 1 ? (mr + 1) / 2 : 0;
+    while (mr > 1 && qms_lds(mr, p.K, p.K >> p.gs_log2, parts, qms_waves(p.K)).total > LDS_PER_CU)
+        mr = (mr + 1) / 2;
     return mr;
 }
 
@@ -826,23 +823,23 @@ template <typename T, int EPI>
 int launch_typed(const QParams &p, int bits, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
         // The few-token kernel from three tokens (4-bit) or two (8-bit), and for
-        // 8-bit rows past K = 4096 at one; a function of M, K and the width, so
-        // every epilogue at one shape adds alike. Measured (us, N x K; before /
+        // 8-bit rows past K = 4096 at one; a function of M, K, the width and the
+        // group size, so every epilogue at one shape adds alike. Measured (us, N x K; before /
         // with it): 4-bit, 9728 x 2560, M = 2 7.2 / 6.5, M = 4 9.6 / 6.8, M = 8 39
         // / 7.2; the dual of it M = 2 10.0 / 11.5, M = 4 14.4 / 11.6; 2560 x 9728,
         // M = 2 7.9 / 8.1, M = 4 38 / 8.4, M = 6 58 / 8.7. 8-bit, 2048 x 8192, M = 1
         // 14.6 / 10.2, M = 6 64 / 11.2; the 8192 x 2048 dual M = 1 9.2 / 10.4, M = 2
         // 17.7 / 10.6, M = 6 27 / 10.7; lm_head (151936 x 2560) M = 1 75 / 77, M = 8
         // 447 / 91.
-        const int mr = p.M == 1 ? 1 : (p.M == 2 ? 2 : 4);
         constexpr int P = epi_parts(EPI);
         const bool few = bits == 4 ? p.M > 2 : (p.M > 1 || p.K > 4096);
-        const int rows = few ? qms_rows(p, EPI) : 0;
-        if (bits == 4 && p.M <= 4 && !rows && qmv_dot2_lds_bytes(mr, p.K) <= 65536)
-            return launch_qmv_dot2<T, EPI>(p, mr, st);
-        if (rows)
+        if (few && qms_takes(p.M, p.K, p.gs_log2)) {
+            const int rows = qms_rows(p, P);
             return bits == 4 ? launch_qms<T, 4, P>(p, EPI, rows, st)
                              : launch_qms<T, 8, P>(p, EPI, rows, st);
+        }
+        if (bits == 4 && p.M <= 2 && qmv_dot2_lds_bytes((int)p.M, p.K) <= 65536)
+            return launch_qmv_dot2<T, EPI>(p, (int)p.M, st);
     }
     return bits == 4 ? launch_qmv<T, 4, EPI>(p, st) : launch_qmv<T, 8, EPI>(p, st);
 }

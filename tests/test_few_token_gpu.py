@@ -80,9 +80,47 @@ def test_few_token_split_and_grouped(bits, D):
         assert torch.equal(got, ops.quantized_matmul(xd, *p, bits=bits))
 
 
+# K between what one part's scales leave room for in the LDS and what two or
+# three parts' do: all epilogues of a shape take one kernel. (fp16 and thousands
+# of outputs: two orders of summation differ in some of them.)
+@pytest.mark.parametrize("K,gs", [(28672, 32), (49152, 64), (20448, 32)])
+@pytest.mark.parametrize("bits,M", [(4, 3), (8, 5)])
+def test_few_token_epilogues_agree_at_long_rows(K, gs, bits, M):
+    D = 512
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(K + bits)
+    xd = torch.randn((1, M, K), generator=gen, device="cuda").half()
+    w, w2 = (random_quantized(3 * D, K, gen, "cuda", gs, bits, torch.float16) for _ in range(2))
+    t, u = (ops.quantized_matmul(xd, *a, group_size=gs, bits=bits) for a in (w, w2))
+    y1, u1 = ops.qmm_dual(xd, *w, *w2, gs, bits)
+    assert torch.equal(y1, t) and torch.equal(u1, u)
+    c, bx = ops.qmm_split_gate(xd, *w, gs, bits)
+    assert torch.equal(c, t[..., D:2 * D]) and torch.equal(bx, t[..., :D] * t[..., 2 * D:])
+    want = xd.double()[0] @ ops.dequantize(*w, group_size=gs, bits=bits).double().t().contiguous()
+    assert float((t.double() - want).abs().max()) <= 1e-2 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("N,K,bits", [(2033, 320, 4), (2048, 320, 4), (2033, 576, 8)])
+def test_few_token_epilogues_agree_at_unaligned_scales(N, K, bits):
+    """One weight of a pair is a view whose scales and biases lie off a 16-byte
+    boundary, or whose last tile's end does (which no 16-byte DMA can take)."""
+    M = 4
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(N + bits)
+    xd = torch.randn((M, K), generator=gen, device="cuda").half()
+    one, w2 = (random_quantized(n, K, gen, "cuda", 64, bits, torch.float16) for n in (N + 1, N))
+    off = [t[1:] for t in one]
+    t, u = (ops.quantized_matmul(xd, *a, bits=bits) for a in (off, w2))
+    assert torch.equal(t, ops.quantized_matmul(xd, *(a.clone() for a in off), bits=bits))
+    y1, u1 = ops.qmm_dual(xd, *off, *w2, 64, bits)
+    assert torch.equal(y1, t) and torch.equal(u1, u)
+    want = xd.double() @ ops.dequantize(*off, bits=bits).double().t().contiguous()
+    assert float((t.double() - want).abs().max()) <= 1e-2 * float(want.abs().max())
+
+
 def test_few_token_unaligned_scales():
-    """Scales and biases that are views off a 16-byte boundary (the kernel's DMA
-    cannot take them) run the generic kernel."""
+    """Scales and biases that are views off a 16-byte boundary (a value a thread
+    in place of the kernel's 16-byte DMA)."""
     M, N, K = 4, 33, 320
     x = oracle.round_to(rng(5200).normal(0, 1, (M, K)), "bfloat16")
     host, w = _dev(5201, N, K, 64, 4, "bfloat16")
