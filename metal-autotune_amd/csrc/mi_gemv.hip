@@ -365,11 +365,12 @@ __global__ __launch_bounds__(WIDE ? 1024 : 256) void qmv_dot2_kernel(QParams p) 
 
 // ---------------------------------------------------------------------------
 // Few-token GEMM (M <= 8, 16-bit T, both widths): the factored per-group sum on
-// the matrix cores. The codes enter v_mfma_f32_16x16x32 exactly (8-bit as the
-// integers 0..255 in bf16, or 1024 + q in fp16; 4-bit as MAG + q, see Magic), x
-// as it is, so a group's D = sum x (MAG + q) and X = sum x (a product with
-// ones) are fp32 sums of exact products, and the row adds s D + (b - MAG s) X
-// per group: the arithmetic of the dot2 GEMV, up to 16 tokens at the cost of one.
+// the matrix cores. The codes enter v_mfma_f32_16x16x32 exactly, as the integers
+// they are, and x as it is, so a group's D = sum x q and X = sum x (a product
+// with ones) are fp32 sums of exact products, and the row adds s D + b X per
+// group, up to 16 tokens at the cost of one. (Codes with an offset, as the dot2
+// GEMV takes them, are cheaper to make and cost the sums three to ten bits: the
+// offset's share has to cancel again.)
 //
 // A workgroup owns 16 output features (per part) and its waves split K in
 // contiguous runs; the partial sums meet in LDS. Operands: A = x (row = token
@@ -398,32 +399,46 @@ template <typename T> __device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f
                                                       __builtin_bit_cast(V8, b), c, 0, 0, 0);
 }
 
-// Eight codes as T: 4 bits, word w0: MAG + q in the order (0, 4), (1, 5), (2, 6),
-// (3, 7); 8 bits, words w0 and w1 in order: q (bf16) or 1024 + q (fp16).
+// Eight codes as T, in order: the nibbles of w0 (4 bits) or the bytes of w0 and w1.
+// 4 bits: a byte below 16 read as an fp8 (E4M3) number is itself 2^-9, through its
+// subnormals and its first binade, so the scaled conversion to a pair of T is two
+// codes an instruction (8 tokens, 9728 x 9728, 4 bits: through fp32, a code an
+// instruction, the dual took 15 to 20 % longer).
+// 8 bits, bf16: an integer below 256 has at most 8 significant bits, so its fp32
+// value's high half is it. fp16: q 2^-24, the subnormal whose bits q is (the
+// caller scales by code_scale, exact).
 template <typename T, int BITS>
 __device__ __forceinline__ uint4 code_frag(uint32_t w0, uint32_t w1) {
     if constexpr (BITS == 4) {
-        return make_uint4(magic_pair<T>(w0, 0), magic_pair<T>(w0, 1), magic_pair<T>(w0, 2),
-                          magic_pair<T>(w0, 3));
+        const uint32_t even = w0 & 0x0F0F0F0Fu, odd = (w0 >> 4) & 0x0F0F0F0Fu;
+        const uint32_t lo = __builtin_amdgcn_perm(odd, even, 0x05010400u);  // codes 0 .. 3
+        const uint32_t hi = __builtin_amdgcn_perm(odd, even, 0x07030602u);  // codes 4 .. 7
+        if constexpr (__is_same(T, bf16))
+            return make_uint4(
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true)));
+        else
+            return make_uint4(
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(lo, 512.0f, true)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, false)),
+                __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(hi, 512.0f, true)));
     } else if constexpr (__is_same(T, bf16)) {
-        // an integer below 256 has at most 8 significant bits: the fp32 value's
-        // high half is it exactly
         auto pair = [](uint32_t w, int sh) {
             return __builtin_amdgcn_perm(__float_as_uint((float)((w >> (sh + 8)) & 255u)),
                                          __float_as_uint((float)((w >> sh) & 255u)), 0x07060302u);
         };
         return make_uint4(pair(w0, 0), pair(w0, 16), pair(w1, 0), pair(w1, 16));
     } else {
-        // bytes (e, q1, e, q0) with e the exponent byte of 1024
-        auto pair = [](uint32_t w, uint32_t sel) {
-            return __builtin_amdgcn_perm(0x64646464u, w, sel);
-        };
+        auto pair = [](uint32_t w, uint32_t sel) { return __builtin_amdgcn_perm(0u, w, sel); };
         return make_uint4(pair(w0, 0x04010400u), pair(w0, 0x04030402u), pair(w1, 0x04010400u),
                           pair(w1, 0x04030402u));
     }
 }
-template <typename T, int BITS> constexpr float code_offset() {
-    return BITS == 4 ? Magic<T>::value : (__is_same(T, bf16) ? 0.0f : 1024.0f);
+template <typename T, int BITS> constexpr float code_scale() {
+    return BITS == 8 && __is_same(T, f16) ? 16777216.0f : 1.0f;
 }
 
 template <int BITS, int P, int GSL, bool PAIR> struct QmsShape {
@@ -480,7 +495,7 @@ template <int P> __device__ __forceinline__ Bound bind_of(const QParams &p, int 
 
 template <typename T, int BITS, int P, int GSL, bool PAIR>
 __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, int nw, int run,
-                                                   int longer) {
+                                                   int longer, int sb_dma) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef QmsShape<BITS, P, GSL, PAIR> Sh;
     typedef __attribute__((address_space(3))) void *lds_ptr;
@@ -499,8 +514,8 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
     char *sbl = qlds + rows * L.pitch;  // [part][scale, bias][16][G]
 
     // x rows, then the scale and bias rows, 16 bytes a lane; the instructions
-    // are dealt to the waves. Scale and bias rows off a 16-byte boundary, or
-    // whose last tile ends off one, come a value a thread.
+    // are dealt to the waves. (sb_dma 0: scale or bias rows off a 16-byte
+    // boundary, or whose last tile ends off one, come a value a thread.)
     {
         const __amdgpu_buffer_rsrc_t xr =
             buffer_rsrc((const T *)p.x + m0 * K, (uint32_t)(rows * K * (int64_t)sizeof(T)));
@@ -518,22 +533,25 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
         const int chunks = 2 * G, ips = (chunks + 63) >> 6;
         const int64_t left = (bd.Nout - nb) * G * 2;  // the part's rows from nb on
         const uint32_t bytes = (uint32_t)(left < L.sb ? left : L.sb);
+        auto sb_rows = [&](int a) {
+            return (const T *)((a & 1) ? bd.b(a >> 1) : bd.s(a >> 1)) + (bd.noff(a >> 1) + nb) * G;
+        };
+        if (sb_dma) {
 #pragma unroll
-        for (int a = 0; a < 2 * P; ++a) {
-            const T *base = (const T *)((a & 1) ? bd.b(a >> 1) : bd.s(a >> 1)) + (bd.noff(a >> 1) + nb) * G;
-            if ((((uintptr_t)base | bytes) & 15) != 0) {  // (workgroup-uniform)
-                T *dst = (T *)(sbl + a * L.sb);
-                for (int i = threadIdx.x; i < (int)(bytes / sizeof(T)); i += 64 * nw) dst[i] = base[i];
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // before the barrier below
-                continue;
+            for (int a = 0; a < 2 * P; ++a) {
+                const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(sb_rows(a), bytes);
+                for (int j = wave; j < ips; j += nw) {
+                    const int c = 64 * j + lane;
+                    if (c < chunks)
+                        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                            sr, (lds_ptr)(sbl + a * L.sb + j * 1024), 16, 16 * c, 0, 0, 0);
+                }
             }
-            const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(base, bytes);
-            for (int j = wave; j < ips; j += nw) {
-                const int c = 64 * j + lane;
-                if (c < chunks)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                        sr, (lds_ptr)(sbl + a * L.sb + j * 1024), 16, 16 * c, 0, 0, 0);
-            }
+        } else {
+            for (int a = 0; a < 2 * P; ++a)
+                for (int i = threadIdx.x; i < (int)(bytes / sizeof(T)); i += 64 * nw)
+                    ((T *)(sbl + a * L.sb))[i] = sb_rows(a)[i];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // before the barrier below
         }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -630,28 +648,21 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
                 for (int q = 0; q < P; ++q) D[q] = zero;
 #pragma unroll
                 for (int st = 0; st < STEPS; ++st) {
-                    uint4 x = a[st];
-                    if constexpr (BITS == 4)  // the codes' order
-                        x = make_uint4(__builtin_amdgcn_perm(x.z, x.x, 0x05040100u),
-                                       __builtin_amdgcn_perm(x.z, x.x, 0x07060302u),
-                                       __builtin_amdgcn_perm(x.w, x.y, 0x05040100u),
-                                       __builtin_amdgcn_perm(x.w, x.y, 0x07060302u));
-                    X = mma16<T>(x, ones, X);
+                    X = mma16<T>(a[st], ones, X);
 #pragma unroll
                     for (int q = 0; q < P; ++q) {
                         const uint32_t *wq = w[i][q] + v * WPL;
-                        D[q] = mma16<T>(x, BITS == 4 ? code_frag<T, BITS>(wq[st], 0u)
+                        D[q] = mma16<T>(a[st], BITS == 4 ? code_frag<T, BITS>(wq[st], 0u)
                                                      : code_frag<T, BITS>(wq[2 * st], wq[2 * st + 1]),
                                         D[q]);
                     }
                 }
 #pragma unroll
                 for (int q = 0; q < P; ++q) {
-                    const float s = (float)sc[q];
-                    const float bb = __builtin_fmaf(-code_offset<T, BITS>(), s, (float)bi[q]);
+                    const float s = (float)sc[q] * code_scale<T, BITS>(), b = (float)bi[q];
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        acc[q][e] = __builtin_fmaf(s, D[q][e], __builtin_fmaf(bb, X[e], acc[q][e]));
+                        acc[q][e] = __builtin_fmaf(s, D[q][e], __builtin_fmaf(b, X[e], acc[q][e]));
                 }
             }
             if (u + GB < u1) load(i, u + GB);
@@ -792,17 +803,29 @@ inline int qms_rows(const QParams &p, int parts) {
     return mr;
 }
 
+// Whether 16-byte DMA takes the scale and bias rows of every tile.
+inline bool qms_sb_dma(const QParams &p, int epi) {
+    const int64_t G = p.K >> p.gs_log2;
+    for (int i = 0; i < 3; ++i) {
+        const int64_t rows = epi == EPI_GROUP3 ? p.pn[i] : p.Nout;
+        if (!aligned(p.s[i], 16) || !aligned(p.b[i], 16) || (p.noff[i] * G) % 8 || (rows * G) % 8)
+            return false;
+    }
+    return true;
+}
+
 template <typename T, int BITS, int P, int GSL>
 void launch_qms_gs(const QParams &p, int epi, int mr, dim3 grid, size_t lds, hipStream_t st) {
-    const int G = (int)(p.K >> GSL), nw = qms_waves(p.K);
+    const int G = (int)(p.K >> GSL), nw = qms_waves(p.K), dma = qms_sb_dma(p, epi);
     if constexpr (qms_pairs<BITS, GSL>()) {
         if (G % 2 == 0) {
-            qms_kernel<T, BITS, P, GSL, true><<<grid, 64 * nw, lds, st>>>(p, epi, mr, nw, G / 2 / nw,
-                                                                          G / 2 % nw);
+            qms_kernel<T, BITS, P, GSL, true><<<grid, 64 * nw, lds, st>>>(
+                p, epi, mr, nw, G / 2 / nw, G / 2 % nw, dma);
             return;
         }
     }
-    qms_kernel<T, BITS, P, GSL, false><<<grid, 64 * nw, lds, st>>>(p, epi, mr, nw, G / nw, G % nw);
+    qms_kernel<T, BITS, P, GSL, false><<<grid, 64 * nw, lds, st>>>(p, epi, mr, nw, G / nw, G % nw,
+                                                                   dma);
 }
 
 template <typename T, int BITS, int P>

@@ -128,6 +128,29 @@ def test_few_token_unaligned_scales():
     _close(y, oracle.qmm_factored(x, *(a[1:] for a in host), 64, 4, "bfloat16"))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bits,M,gs", [(4, 3, 64), (4, 5, 32), (4, 8, 128), (8, 2, 64), (8, 6, 32),
+                                       (8, 8, 128)])
+def test_few_token_sums_hold_small_products(bits, M, gs, dtype):
+    """Every group's one code that is not zero meets a small x: sum x q is that
+    product, and every partial sum of such products is exact in fp32, whatever
+    the other, large x are. (Codes with an offset sum the large x as well, and
+    lose the small product in their last bits.)"""
+    N, K = 64, 8 * gs
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M)
+    x = (1 + torch.rand((M, K), generator=gen, device="cuda")).to(dtype)
+    x[:, ::gs] = 2.0 ** -12
+    w = torch.zeros((N, K * bits // 32), dtype=torch.int32, device="cuda")
+    w[:, ::gs * bits // 32] = 3                       # the group's first code
+    s = torch.ones((N, K // gs), dtype=dtype, device="cuda")
+    b = torch.zeros_like(s)
+    want = torch.full((M, N), 8 * 3 * 2.0 ** -12, device="cuda").to(dtype)
+    assert torch.equal(ops.quantized_matmul(x, w, s, b, group_size=gs, bits=bits), want)
+    y1, y2 = ops.qmm_dual(x, w, s, b, w, s, b, gs, bits)
+    assert torch.equal(y1, want) and torch.equal(y2, want)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("M", [1, 3, 8])
 def test_generic_kernel_epilogues_agree(M, bits):
