@@ -34,8 +34,8 @@ __device__ __forceinline__ void load_x(const T *xp, float (&xf)[VPC]) {
 }
 
 // a b + c d with the rounding written out: left to contraction, the compiler
-// fused one product or the other by the epilogue it compiled, and an epilogue's
-// fp32 sums differed from the plain projection's in their last bit.
+// fuses one product or the other, and an epilogue's fp32 sums may differ from the
+// plain projection's in their last bit.
 __device__ __forceinline__ float fma_mul(float a, float b, float c, float d) {
 #pragma clang fp contract(off)
     return __builtin_fmaf(a, b, c * d);
@@ -103,7 +103,14 @@ __global__ __launch_bounds__(256) void qmv_kernel(QParams p) {
                 float dq = 0.0f;
 #pragma unroll
                 for (int i = 0; i < VPC; ++i) dq = __builtin_fmaf(xf[i], qf[q][i], dq);
-                acc[q][m] += fma_mul(bi[q], dx, sc[q], dq);
+                // every instance rounds this as fma(bi, dx, sc dq): left to
+                // contraction, all but the split(3) ones at 4 bits do. (Written
+                // out everywhere, the compiler sinks the weight loads to their
+                // use: 8-bit dual, one token, 7656 x 1792 8.2 -> 17.4 us.)
+                if constexpr (P == 3 && BITS == 4)
+                    acc[q][m] += fma_mul(bi[q], dx, sc[q], dq);
+                else
+                    acc[q][m] += sc[q] * dq + bi[q] * dx;
             }
         }
     }
@@ -402,8 +409,8 @@ template <typename T> __device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f
 // Eight codes as T, in order: the nibbles of w0 (4 bits) or the bytes of w0 and w1.
 // 4 bits: a byte below 16 read as an fp8 (E4M3) number is itself 2^-9, through its
 // subnormals and its first binade, so the scaled conversion to a pair of T is two
-// codes an instruction (8 tokens, 9728 x 9728, 4 bits: through fp32, a code an
-// instruction, the dual took 15 to 20 % longer).
+// codes an instruction (through fp32, a code an instruction, the 8848 x 9728 dual
+// at 4 tokens took 44.5 us, not 36.4).
 // 8 bits, bf16: an integer below 256 has at most 8 significant bits, so its fp32
 // value's high half is it. fp16: q 2^-24, the subnormal whose bits q is (the
 // caller scales by code_scale, exact).

@@ -152,7 +152,7 @@ def test_few_token_sums_hold_small_products(bits, M, gs, dtype):
 
 
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("M", [1, 2, 3, 8])
 def test_generic_kernel_epilogues_agree(M, bits):
     """The fp32 kernel's sums are its outputs: an epilogue that rounds a group's
     sum in another way shows in the last bit."""
@@ -166,3 +166,6 @@ def test_generic_kernel_epilogues_agree(M, bits):
     assert torch.equal(y1, t) and torch.equal(u1, u)
     c, bx = ops.qmm_split_gate(xd, *w, 64, bits)
     assert torch.equal(c, t[..., 32:64]) and torch.equal(bx, t[..., :32] * t[..., 64:])
+    assert torch.equal(ops.qmm_residual(xd, *w, torch.zeros_like(t), 64, bits), t)
+    for y, a in zip(ops.qmm_grouped3(xd, (w, w2, w), 64, bits), (t, u, t)):
+        assert torch.equal(y, a)
