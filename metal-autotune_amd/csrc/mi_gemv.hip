@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void qmv_kernel(QParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Decode GEMV (M <= 2, 4-bit, bf16/fp16): the nibbles never go through a
+// Decode GEMV (M <= 2, up to K = 512 M <= 4; 4-bit, bf16/fp16): the nibbles never go through a
 // float conversion. (w >> 4j) & 0x000F000F | MAGIC packs nibbles j and j+4 of a
 // word as the two 16-bit floats MAG + q exactly (bf16: 0x4300 = 128, ulp 1 up
 // to 256; fp16: 0x6400 = 1024, ulp 1), so one v_and_or makes a pair and
@@ -395,6 +395,10 @@ __global__ __launch_bounds__(WIDE ? 1024 : 256) void qmv_dot2_kernel(QParams p) 
 // swaps) lost: the registers it held left one workgroup a CU (12.4 us).
 // Otherwise a unit is one group, a quarter a lane.
 //
+// A unit's scales and biases are read together: two 2-byte LDS reads a part and
+// group had bound the narrow groups (dual 9728 x 2048, 4 tokens, group 32 21.2 ->
+// 10.7 us; x 4096, group 64 20.7 -> 16.6).
+//
 // Bound: HBM, one memory round trip after the launch.
 template <typename T> __device__ __forceinline__ f32x4 mma16(uint4 a, uint4 b, f32x4 c) {
     typedef typename Vec<T>::x8 V8;
@@ -454,7 +458,10 @@ template <int BITS, int P, int GSL, bool PAIR> struct QmsShape {
     static constexpr int U = PAIR ? 2 : 1;                    // groups per unit
     static constexpr int UW = WPL * U;                        // words per lane and unit
     static constexpr int FIT = (P == 3 ? 24 : 48) / (UW * P);
-    static constexpr int GB = FIT > 8 / U ? 8 / U : (FIT < 1 ? 1 : FIT);  // units in flight
+    // units in flight: 8 groups, 6 where a second part at group 32 takes the
+    // registers (8: 3 to 5 % slower at K = 4096)
+    static constexpr int CAP = GSL == 5 && BITS == 4 && P == 2 ? 3 : 8 / U;
+    static constexpr int GB = FIT > CAP ? CAP : (FIT < 1 ? 1 : FIT);
 };
 template <int BITS, int GSL> constexpr bool qms_pairs() {
     return QmsShape<BITS, 1, GSL, false>::WPL <= 2;
@@ -637,19 +644,26 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
                         w[i][q][j] = r[0], w[i][q][WPL + j] = r[1];
                     }
             }
+            // the unit's scales and biases (PAIR: both groups' in one read)
+            T sc[P][U], bi[P][U];
+#pragma unroll
+            for (int q = 0; q < P; ++q) {
+                const char *ps = sp + (2 * q) * L.sb + 2 * U * u, *pb = ps + L.sb;
+                if constexpr (PAIR) {
+                    typedef T T2 __attribute__((ext_vector_type(2)));
+                    const T2 s2 = *(const T2 *)ps, b2 = *(const T2 *)pb;
+                    sc[q][0] = s2.x, sc[q][1] = s2.y, bi[q][0] = b2.x, bi[q][1] = b2.y;
+                } else {
+                    sc[q][0] = *(const T *)ps, bi[q][0] = *(const T *)pb;
+                }
+            }
 #pragma unroll
             for (int v = 0; v < U; ++v) {
                 const int g = U * u + v;
                 uint4 a[STEPS];
-                T sc[P], bi[P];
 #pragma unroll
                 for (int st = 0; st < STEPS; ++st)
                     a[st] = *(const uint4 *)(xp + (g << (GSL + 1)) + 16 * st);
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    sc[q] = *(const T *)(sp + (2 * q) * L.sb + 2 * g);
-                    bi[q] = *(const T *)(sp + (2 * q + 1) * L.sb + 2 * g);
-                }
                 f32x4 X = zero, D[P];
 #pragma unroll
                 for (int q = 0; q < P; ++q) D[q] = zero;
@@ -666,7 +680,7 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
                 }
 #pragma unroll
                 for (int q = 0; q < P; ++q) {
-                    const float s = (float)sc[q] * code_scale<T, BITS>(), b = (float)bi[q];
+                    const float s = (float)sc[q][v] * code_scale<T, BITS>(), b = (float)bi[q][v];
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
                         acc[q][e] = __builtin_fmaf(s, D[q][e], __builtin_fmaf(b, X[e], acc[q][e]));
@@ -764,8 +778,10 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
     } else if (!row_wave && waves == 4) {
         if (mr == 1)
             qmv_dot2_kernel<T, 1, EPI><<<grid, bs, lds, st>>>(p);
-        else
+        else if (mr == 2)
             qmv_dot2_kernel<T, 2, EPI><<<grid, bs, lds, st>>>(p);
+        else
+            qmv_dot2_kernel<T, 4, EPI><<<grid, bs, lds, st>>>(p);
     } else if constexpr (wide_ok) {
         // a row a wave takes PF too at M = 1 while x fits two chunks a thread
         // (Qwen3's down_proj at decode, 10-wave workgroups: 6.7 -> 5.6 us)
@@ -787,8 +803,10 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
         } else {
             if (mr == 1)
                 qmv_dot2_kernel<T, 1, EPI, false, true><<<grid, bs, lds, st>>>(p);
-            else
+            else if (mr == 2)
                 qmv_dot2_kernel<T, 2, EPI, false, true><<<grid, bs, lds, st>>>(p);
+            else
+                qmv_dot2_kernel<T, 4, EPI, false, true><<<grid, bs, lds, st>>>(p);
         }
     }
     return launch_status("quantized matmul (dot2 qmv)");
@@ -854,22 +872,28 @@ int launch_typed(const QParams &p, int bits, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
         // The few-token kernel from three tokens (4-bit) or two (8-bit), and for
         // 8-bit rows past K = 4096 at one; a function of M, K, the width and the
-        // group size, so every epilogue at one shape adds alike. Measured (us, N x K; before /
-        // with it): 4-bit, 9728 x 2560, M = 2 7.2 / 6.5, M = 4 9.6 / 6.8, M = 8 39
-        // / 7.2; the dual of it M = 2 10.0 / 11.5, M = 4 14.4 / 11.6; 2560 x 9728,
-        // M = 2 7.9 / 8.1, M = 4 38 / 8.4, M = 6 58 / 8.7. 8-bit, 2048 x 8192, M = 1
-        // 14.6 / 10.2, M = 6 64 / 11.2; the 8192 x 2048 dual M = 1 9.2 / 10.4, M = 2
-        // 17.7 / 10.6, M = 6 27 / 10.7; lm_head (151936 x 2560) M = 1 75 / 77, M = 8
-        // 447 / 91.
+        // group size, so every epilogue at one shape adds alike. Measured (us, N x
+        // K; the GEMVs / it): 4-bit, 9728 x 2560, M = 2 7.2 / 6.5, M = 4 9.8 / 6.3,
+        // M = 8 34 / 6.7; the dual of it M = 2 10.0 / 11.5, M = 4 13.3 / 10.2; 2560 x
+        // 9728, M = 2 7.9 / 8.1, M = 4 27 / 7.5, M = 6 50 / 8.0. 8-bit, 2048 x 8192,
+        // M = 1 11.4 / 10.1, M = 6 58 / 11.1, but 5040 x 5120, M = 1 9.0 / 10.6; the
+        // 8192 x 2048 dual M = 1 9.4 / 10.4, M = 2 13.9 / 8.9, M = 6 24 / 9.0; lm_head
+        // (151936 x 2560) M = 1 71 / 77, M = 8 445 / 92.
+        // Short rows stay with the GEMVs, which have less to set up: 8-bit M = 2,
+        // 8192 x 768 3.6 / 4.2, 892 x 1024 4.8 / 4.4, M = 3, 944 x 256 2.7 / 3.2, x 768
+        // 4.2 / 3.4; 4-bit M = 3, 2048 x 512 3.1 / 3.3, x 768 3.7 / 3.6.
         constexpr int P = epi_parts(EPI);
-        const bool few = bits == 4 ? p.M > 2 : (p.M > 1 || p.K > 4096);
-        if (few && qms_takes(p.M, p.K, p.gs_log2)) {
+        const int64_t M = p.M;
+        const bool few = bits == 4 ? M > 4 || (M > 2 && p.K > 512)
+                                   : p.K > (M == 1 ? 4096 : M == 2 ? 768 : 256);
+        if (few && qms_takes(M, p.K, p.gs_log2)) {
             const int rows = qms_rows(p, P);
             return bits == 4 ? launch_qms<T, 4, P>(p, EPI, rows, st)
                              : launch_qms<T, 8, P>(p, EPI, rows, st);
         }
-        if (bits == 4 && p.M <= 2 && qmv_dot2_lds_bytes((int)p.M, p.K) <= 65536)
-            return launch_qmv_dot2<T, EPI>(p, (int)p.M, st);
+        const int mr = M > 2 ? 4 : (int)M;
+        if (bits == 4 && M <= 4 && qmv_dot2_lds_bytes(mr, p.K) <= 65536)
+            return launch_qmv_dot2<T, EPI>(p, mr, st);
     }
     return bits == 4 ? launch_qmv<T, 4, EPI>(p, st) : launch_qmv<T, 8, EPI>(p, st);
 }

@@ -136,7 +136,7 @@ def test_few_token_sums_hold_small_products(bits, M, gs, dtype):
     product, and every partial sum of such products is exact in fp32, whatever
     the other, large x are. (Codes with an offset sum the large x as well, and
     lose the small product in their last bits.)"""
-    N, K = 64, 8 * gs
+    N, K = 64, 32 * gs
     gen = torch.Generator(device="cuda")
     gen.manual_seed(M)
     x = (1 + torch.rand((M, K), generator=gen, device="cuda")).to(dtype)
@@ -145,7 +145,7 @@ def test_few_token_sums_hold_small_products(bits, M, gs, dtype):
     w[:, ::gs * bits // 32] = 3                       # the group's first code
     s = torch.ones((N, K // gs), dtype=dtype, device="cuda")
     b = torch.zeros_like(s)
-    want = torch.full((M, N), 8 * 3 * 2.0 ** -12, device="cuda").to(dtype)
+    want = torch.full((M, N), 32 * 3 * 2.0 ** -12, device="cuda").to(dtype)
     assert torch.equal(ops.quantized_matmul(x, w, s, b, group_size=gs, bits=bits), want)
     y1, y2 = ops.qmm_dual(x, w, s, b, w, s, b, gs, bits)
     assert torch.equal(y1, want) and torch.equal(y2, want)
