@@ -103,12 +103,15 @@ template <int D> __device__ __forceinline__ void attn_init(AttnState<D> &st) {
     st.l = 0.0f;
 }
 
-// The larger of a lane's value and that of the lane 32 away, in both.
+// The larger of a lane's value and that of the lane 32 away, in both. (The pair's
+// members are copied out first: a bit cast of a vector's subscript reads its first
+// element, whatever the subscript.)
 __device__ __forceinline__ float max_halves(float v) {
     typedef unsigned U2 __attribute__((ext_vector_type(2)));
     const unsigned u = __builtin_bit_cast(unsigned, v);
     const U2 r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
-    return fmaxf(__builtin_bit_cast(float, r[0]), __builtin_bit_cast(float, r[1]));
+    const unsigned lo = r[0], hi = r[1];
+    return fmaxf(__builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi));
 }
 
 // Scores of keys from `vis` on (of the tile's 32) set to -inf.

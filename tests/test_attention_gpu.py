@@ -81,3 +81,29 @@ def test_sdpa_without_a_workspace(Lq, Lk):
     assert torch.equal(o, o1)
     _close(o, oracle.sdpa(*(to_np(x) for x in t), D ** -0.5, True, "bfloat16"))
     _close(ops.scaled_dot_product_attention(q, k, v, D ** -0.5), to_np(o).astype(np.float64))
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("H,HK,Lq,Lk,D", [
+    (8, 2, 1, 128, 128),      # decode
+    (8, 2, 2, 2048, 64),      # ... split
+    (8, 2, 32, 160, 64),      # few query rows
+    (32, 8, 400, 512, 128),   # shared tiles
+])
+@pytest.mark.parametrize("gap", [25.0, 150.0])
+def test_sdpa_one_large_score(H, HK, Lq, Lk, D, gap, dtype):
+    """One key's score lies far above the others', at each position of a key
+    tile in turn: its value is the result (the other weights are below 2^-36),
+    and no exponent overflows, whichever lane holds that score."""
+    tdt = getattr(torch, dtype)
+    q = torch.zeros((1, H, Lq, D), device="cuda")
+    q[..., 0] = 1
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(7)
+    v = torch.randn((1, HK, Lk, D), generator=gen, device="cuda").to(tdt)
+    for pos in [*range(32), 32 + 4, Lk - 1]:
+        k = torch.zeros((1, HK, Lk, D), device="cuda")
+        k[:, :, pos, 0] = 1
+        o = ops.scaled_dot_product_attention(q.to(tdt), k.to(tdt), v, gap, None)
+        want = v[:, :, pos].repeat_interleave(H // HK, 1)[:, :, None].expand_as(o)
+        assert bool(((o.float() - want.float()).abs() <= 2 ** -7 * want.float().abs() + 1e-6).all()), pos
