@@ -63,21 +63,10 @@ template <> struct AMfma<bf16> {
     static __device__ __forceinline__ f32x16 mma(bf16x8 a, bf16x8 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
-    // c plus the two values of a packed pair, in fp32
-    static __device__ __forceinline__ float add_pair(uint32_t p, float c) {
-        typedef __bf16 v2 __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2, p),
-                                               __builtin_bit_cast(v2, 0x3F803F80u), c, false);
-    }
 };
 template <> struct AMfma<f16> {
     static __device__ __forceinline__ f32x16 mma(f16x8 a, f16x8 b, f32x16 c) {
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ float add_pair(uint32_t p, float c) {
-        typedef _Float16 v2 __attribute__((ext_vector_type(2)));
-        return __builtin_amdgcn_fdot2(__builtin_bit_cast(v2, p),
-                                      __builtin_bit_cast(v2, 0x3C003C00u), c, false);
     }
 };
 
@@ -124,9 +113,9 @@ __device__ __forceinline__ void attn_mask(f32x16 &s, int vis, int h2) {
 // Scores to probabilities of one key tile: s[i] = S^T (key 8*(i/4) + 4*h2 +
 // i%4 of the tile, the lane's query row; -inf where the row does not see the
 // key), pk gets 2^(s scale - m) in pairs of T, in register order. The row sum
-// adds those rounded values, the ones the PV product uses, so a row's weights
-// sum to one (and a pair is one dot2). scale > 0 (a negative scale was moved
-// into Q's sign).
+// adds the fp32 values, in four chains (rounded to T first, the denominator
+// would carry T's error of a probability, up to 2^-8 in bf16). scale > 0 (a
+// negative scale was moved into Q's sign).
 template <typename T, int D>
 __device__ __forceinline__ void attn_softmax(AttnState<D> &st, const f32x16 &s, uint32_t (&pk)[8],
                                              float scale) {
@@ -153,14 +142,17 @@ __device__ __forceinline__ void attn_softmax(AttnState<D> &st, const f32x16 &s, 
     }
     // (a row that has seen no key yet: every score is -inf, and p is 0)
     const float nm = st.m == -INFINITY ? 0.0f : -st.m;
-    float psum = 0.0f;
+    float sum[4];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        pk[i] = pk2<T>(__builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i], scale, nm)),
-                       __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i + 1], scale, nm)));
-        psum = AMfma<T>::add_pair(pk[i], psum);
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i], scale, nm));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * i + 1], scale, nm));
+        pk[i] = pk2<T>(p0, p1);
+        float &a = sum[2 * (i & 1)], &b = sum[2 * (i & 1) + 1];
+        a = i < 2 ? p0 : a + p0;
+        b = i < 2 ? p1 : b + p1;
     }
-    st.l += psum;
+    st.l += (sum[0] + sum[1]) + (sum[2] + sum[3]);
 }
 
 // Swizzles of a staged tile: 16-byte chunk c of key row r sits at chunk

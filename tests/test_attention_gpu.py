@@ -107,3 +107,31 @@ def test_sdpa_one_large_score(H, HK, Lq, Lk, D, gap, dtype):
         o = ops.scaled_dot_product_attention(q.to(tdt), k.to(tdt), v, gap, None)
         want = v[:, :, pos].repeat_interleave(H // HK, 1)[:, :, None].expand_as(o)
         assert bool(((o.float() - want.float()).abs() <= 2 ** -7 * want.float().abs() + 1e-6).all()), pos
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("H,HK,Lq,Lk,D", [
+    (8, 2, 1, 992, 128),      # decode
+    (8, 2, 2, 2048, 64),      # ... split
+    (8, 2, 32, 160, 64),      # few query rows
+    (32, 8, 400, 512, 128),   # shared tiles
+])
+def test_sdpa_row_sum_adds_unrounded_weights(H, HK, Lq, Lk, D, dtype):
+    """In every tile of 32 keys one has weight 1 and value 1, the others weight p
+    and value 0, with p just below the middle between two values of the type:
+    the result is 1 / (1 + 31 p), correctly rounded; with the rounded p in the
+    sum it is the next value up."""
+    half_step = 2.0 ** (-9 if dtype == "bfloat16" else -12)
+    p = 0.5 + 0.95 * half_step
+    q = torch.zeros((1, H, Lq, D), device="cuda")
+    q[..., 0] = 1
+    k = torch.zeros((1, HK, Lk, D), device="cuda")
+    k[..., 0] = 1
+    v = torch.zeros_like(k)
+    k[:, :, ::32] = 0
+    v[:, :, ::32] = 1
+    tdt = getattr(torch, dtype)
+    o = ops.scaled_dot_product_attention(q.to(tdt), k.to(tdt), v.to(tdt), float(np.log(p)), None)
+    want = torch.tensor(1 / (1 + 31 * p), dtype=torch.float64).to(tdt)
+    assert torch.tensor(1 / (1 + 31 * 0.5), dtype=torch.float64).to(tdt) != want
+    assert bool((o == want.cuda()).all()), (float(o.min()), float(o.max()), float(want))
