@@ -39,8 +39,9 @@
 // j <= i + Lk - Lq) and key tiles past the last visible key are skipped.
 // A row's result depends only on its global position and the keys, so a
 // chunked prefill whose chunks start at multiples of 32 reproduces the whole
-// prefill bit for bit, and a decode call over at most DEC_SPLIT_MIN_LK keys the
-// last prefill row.
+// prefill bit for bit, and a decode call the last prefill row; except that split
+// calls (at most DEC_MAX_LQ rows over more than DEC_SPLIT_MIN_LK keys, with a
+// workspace), a short last chunk among them, agree within rounding.
 //
 // What bounds it: at long prompts the softmax VALU, about 65 instructions and
 // 16 v_exp (a quarter-rate unit) for the 16 MFMAs of a tile at D = 128, 8 at D =
@@ -775,9 +776,9 @@ struct AttnArgs {
 // Splits of a decode call and key tiles per split (a multiple of four: the
 // streams keep their tiles). One workgroup per split and column block; past
 // DEC_SPLIT_MIN_LK keys as many as put two workgroups on every CU (256), each
-// wave at least one tile. Up to that line one workgroup a kv head: the second
-// launch costs as much as the longer chain (1001 keys unsplit 9.6 us, 1025
-// split 8.1), and a decode row keeps the bits of the prefill's.
+// wave at least one tile. Up to that line one workgroup a kv head, so that a
+// decode row keeps the bits of the prefill's there (by time alone the line would
+// lie lower: 1001 keys unsplit take 9.6 us, 1025 split 8.1).
 struct DecSplit {
     int ncb, nsplit, tps;
 };
@@ -855,8 +856,10 @@ int run_sdpa(const void *q, const void *k, const void *v, void *out, int64_t B, 
     const int64_t need = mi_sdpa_workspace_bytes(B, H, HK, Lq, Lk, D);
     float *w = need > 0 && ws && ws_bytes >= need && aligned(ws, 16) ? (float *)ws : nullptr;
     const float sl = scale * 1.4426950408889634f;
-    // (a scale of 0 as the smallest normal: masked scores stay -inf)
-    const AttnArgs a = {q, k, v, out, B, H, HK, Lq, Lk, kv_cap, fmaxf(fabsf(sl), 1.17549435e-38f),
+    // (a scale of 0 as the smallest normal: masked scores stay -inf; NaN stays
+    // NaN)
+    const float mag = fabsf(sl) < 1.17549435e-38f ? 1.17549435e-38f : fabsf(sl);
+    const AttnArgs a = {q, k, v, out, B, H, HK, Lq, Lk, kv_cap, mag,
                         sl < 0.0f ? 0x80008000u : 0u, causal, out_layout};
     hipStream_t st = as_stream(stream);
     if (dtype == MI_BF16)

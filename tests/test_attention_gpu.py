@@ -135,3 +135,28 @@ def test_sdpa_row_sum_adds_unrounded_weights(H, HK, Lq, Lk, D, dtype):
     want = torch.tensor(1 / (1 + 31 * p), dtype=torch.float64).to(tdt)
     assert torch.tensor(1 / (1 + 31 * 0.5), dtype=torch.float64).to(tdt) != want
     assert bool((o == want.cuda()).all()), (float(o.min()), float(o.max()), float(want))
+
+
+@pytest.mark.parametrize("Lq,Lk", [(1, 40), (2, 1500), (40, 40), (400, 400)])
+def test_sdpa_scale_of_nan(Lq, Lk):
+    q, k = torch.ones((1, 32, Lq, 64), device="cuda").bfloat16(), torch.ones(
+        (1, 8, Lk, 64), device="cuda").bfloat16()
+    assert bool(ops.scaled_dot_product_attention(q, k, k, float("nan")).isnan().all())
+
+
+def test_sdpa_short_last_chunk():
+    """The last 4 of 2052 rows as a call of their own: the whole prefill's bits
+    without a workspace (the same streams), within rounding through ops (split)."""
+    r = rng(4200)
+    H, HK, D, L, tail = 16, 4, 128, 2052, 4
+    q, k, v = (to_torch(oracle.round_to(r.normal(0, 1, (1, h, L, D)), "bfloat16"), "bfloat16")
+               for h in (H, HK, HK))
+    whole = ops.scaled_dot_product_attention(q, k, v, D ** -0.5)[:, :, -tail:]
+    qt = q[:, :, -tail:].contiguous()
+    o = torch.empty_like(qt)
+    assert hip.lib().mi_sdpa(qt.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), 1, H, HK, tail,
+                             L, D, L, D ** -0.5, 1, 0, hip.MI_BF16,
+                             torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(o, whole)
+    split = ops.scaled_dot_product_attention(qt, k, v, D ** -0.5)
+    _close(split, to_np(whole).astype(np.float64))
