@@ -160,7 +160,11 @@ __global__ __launch_bounds__(256) void linear_f32_kernel(const float *__restrict
 // depend on which workgroup finished last. It then resets the counter: the
 // workspace's counters are zero before the first call and after every call.
 // The partials are stored with agent scope (written through) and acknowledged
-// before the ticket, where a release fence writes back the whole XCD's L2.
+// before the ticket, where a release fence writes back the whole XCD's L2. That
+// order rests on the hardware, not on the language's memory model: an agent-scope
+// store bypasses the XCD's L2 (sc1), its vmcnt falls once it is visible to the
+// agent, and the ticket is issued after every wave has waited for that count; the
+// asm's clobber keeps the compiler to the same order.
 // Bound: the chain of launch, W1, W2 (requested under phase 1), ticket and the
 // partials' round trips: 32 x 256 -> 1024 -> 256 54 -> 19 us, 512 rows 196 -> 51.
 constexpr int MLP_HT = 64;      // hidden units per workgroup
@@ -170,6 +174,113 @@ constexpr int64_t MLP_MAX_K = 1024;  // x rows staged in LDS: 8 x 1024 fp32 = 32
 
 __device__ __forceinline__ float gelu_erf(float v) {
     return v * (1.0f + erff(v / 1.41421356237f)) / 2.0f;
+}
+
+// Few rows of a small network (mlp_short): a weight row a lane, and one plain pass
+// over the partials. 5 KB of code against the quad form's 72, which a workgroup
+// with little else to do waits to fetch: 21 rows, 24 -> 20 -> 509 11.3 us against
+// 18.8; 60 rows, 32 -> 104 -> 250 12.4 / 14.5; 5 rows, 80 -> 196 -> 213 13.1 / 13.7.
+// Past the line its chains of dependent loads, and its release fences (an L2
+// writeback a workgroup), cost more: 65 rows, 88 -> 180 -> 442 24.5 / 21.9, 292 rows,
+// 48 -> 184 -> 322 34.6 / 19.9.
+inline bool mlp_short(int64_t M, int64_t K, int64_t H) {
+    return K <= 160 && K * H <= 16384 && (H <= 128 ? M * H <= 6400 : H <= 288 && M <= 8);
+}
+
+__global__ __launch_bounds__(MLP_THREADS) void gelu_mlp_short_f32_kernel(
+    const float *__restrict__ x, const float *__restrict__ w1, const float *__restrict__ b1,
+    const float *__restrict__ w2, const float *__restrict__ b2, float *__restrict__ y,
+    float *__restrict__ part, unsigned *__restrict__ tickets, int64_t M, int64_t K, int64_t H,
+    int64_t N) {
+    extern __shared__ __attribute__((aligned(16))) float mlp_lds[];
+    float *xs = mlp_lds;                       // [MLP_RT][K]
+    float *hs = mlp_lds + MLP_RT * K;          // [MLP_RT][MLP_HT]
+    __shared__ int last;
+    const int t = threadIdx.x;
+    const int64_t c = blockIdx.x, rb = blockIdx.y;
+    const int64_t C = gridDim.x;
+    const int64_t r0 = rb * MLP_RT;
+    const int rows = (int)(M - r0 < MLP_RT ? M - r0 : MLP_RT);
+
+    // stage the row block of x (rows past M read as zero)
+    for (int64_t i = t; i < MLP_RT * K / 4; i += MLP_THREADS) {
+        const int64_t r = (4 * i) / K, k = 4 * i - r * K;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (r < rows) v = *(const float4 *)(x + (r0 + r) * K + k);
+        *(float4 *)(xs + r * K + k) = v;
+    }
+    __syncthreads();
+
+    // phase 1: lane j of wave w computes hidden unit 64 c + j for rows w, w + 4
+    {
+        const int j = t & 63, w = t >> 6;
+        const int64_t hj = c * MLP_HT + j;
+        const int64_t hrow = hj < H ? hj : H - 1;  // clamped, valid row
+        const float *wr = w1 + hrow * K;
+        float a0 = 0.0f, a1 = 0.0f;
+        for (int64_t k = 0; k < K; k += 4) {
+            const float4 wv = *(const float4 *)(wr + k);
+            const float4 xa = *(const float4 *)(xs + w * K + k);
+            const float4 xb = *(const float4 *)(xs + (w + 4) * K + k);
+            a0 = __builtin_fmaf(xa.x, wv.x, a0);
+            a0 = __builtin_fmaf(xa.y, wv.y, a0);
+            a0 = __builtin_fmaf(xa.z, wv.z, a0);
+            a0 = __builtin_fmaf(xa.w, wv.w, a0);
+            a1 = __builtin_fmaf(xb.x, wv.x, a1);
+            a1 = __builtin_fmaf(xb.y, wv.y, a1);
+            a1 = __builtin_fmaf(xb.z, wv.z, a1);
+            a1 = __builtin_fmaf(xb.w, wv.w, a1);
+        }
+        const float bias = b1 ? b1[hrow] : 0.0f;
+        hs[w * MLP_HT + j] = hj < H ? gelu_erf(a0 + bias) : 0.0f;
+        hs[(w + 4) * MLP_HT + j] = hj < H ? gelu_erf(a1 + bias) : 0.0f;
+    }
+    __syncthreads();
+
+    // phase 2: thread t takes output columns n = t, t + 256, ... for all rows
+    const int64_t hbase = c * MLP_HT;
+    const int hn = (int)(H - hbase < MLP_HT ? H - hbase : MLP_HT);  // a multiple of 4
+    float *pc = part + c * (M * N);
+    for (int64_t n = t; n < N; n += MLP_THREADS) {
+        const float *wr = w2 + n * H + hbase;
+        float acc[MLP_RT];
+#pragma unroll
+        for (int r = 0; r < MLP_RT; ++r) acc[r] = 0.0f;
+        for (int hh = 0; hh < hn; hh += 4) {
+            const float4 wv = *(const float4 *)(wr + hh);
+#pragma unroll
+            for (int r = 0; r < MLP_RT; ++r) {
+                const float4 hv = *(const float4 *)(hs + r * MLP_HT + hh);
+                acc[r] = __builtin_fmaf(hv.x, wv.x, acc[r]);
+                acc[r] = __builtin_fmaf(hv.y, wv.y, acc[r]);
+                acc[r] = __builtin_fmaf(hv.z, wv.z, acc[r]);
+                acc[r] = __builtin_fmaf(hv.w, wv.w, acc[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < MLP_RT; ++r)
+            if (r < rows) pc[(r0 + r) * N + n] = acc[r];
+    }
+
+    // phase 3: the last workgroup of this row block reduces the partials
+    __threadfence();  // release: this workgroup's partials before its ticket
+    __syncthreads();
+    if (t == 0) {
+        const unsigned ticket = atomicAdd(&tickets[rb], 1u);
+        last = ticket == (unsigned)(C - 1);
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();  // acquire: every partial of the row block is visible
+    for (int64_t i = t; i < (int64_t)rows * N; i += MLP_THREADS) {
+        const int64_t r = i / N, n = i - r * N;
+        const int64_t o = (r0 + r) * N + n;
+        float s = part[o];
+        for (int64_t cc = 1; cc < C; ++cc) s += part[cc * (M * N) + o];
+        if (b2) s += b2[n];
+        y[o] = s;
+    }
+    if (t == 0) __hip_atomic_store(&tickets[rb], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The sum over a lane's quad, the same bits in its four lanes.
@@ -232,8 +343,8 @@ __device__ __forceinline__ void mlp_reduce_by(const float *part, const float *__
 // A round trip to the partials costs some 2 us, so a thread asks for several
 // pieces at once, and for no more planes than there are: one piece of 16 planes
 // a trip made a row block of 8 x 500 in two planes sixteen trips of 16 loads.
-// 32 rows, 64 -> 128 -> 501 30.4 -> 24.4 us, 1020 -> 2044 -> 509 59 -> 49; 512
-// rows of the latter 252 -> 207, 64 -> 128 -> 501 34 -> 28.
+// 32 rows, 1020 -> 2044 -> 509 59 -> 49 us against that form; 512
+// rows of it 252 -> 207.
 template <int V>
 __device__ __forceinline__ void mlp_reduce(const float *part, const float *__restrict__ b2,
                                            float *__restrict__ y, int rows, int64_t N,
@@ -355,8 +466,9 @@ __global__ __launch_bounds__(MLP_THREADS) void gelu_mlp_f32_kernel(
     }
 
     // phase 3: the last workgroup of this row block reduces the partials
-    __builtin_amdgcn_s_waitcnt(0);  // this wave's partials are at the agent's level ...
-    __syncthreads();                // ... and every wave's, before the ticket
+    // this wave's partials are at the agent's level, after the barrier every wave's
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
     if (t == 0) {
         const unsigned ticket =
             __hip_atomic_fetch_add(&tickets[rb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -700,8 +812,9 @@ extern "C" int mi_gelu_mlp_f32(const float *x, const float *w1, const float *b1,
     float *part = (float *)((char *)workspace + mlp_tickets_bytes());
     const dim3 grid((unsigned)ceil_div(H, MLP_HT), (unsigned)ceil_div(M, MLP_RT));
     const size_t lds = (size_t)(MLP_RT * K + MLP_RT * MLP_HT) * sizeof(float);
-    gelu_mlp_f32_kernel<<<grid, MLP_THREADS, lds, as_stream(stream)>>>(x, w1, b1, w2, b2, y, part,
-                                                                       tickets, M, K, H, N);
+    const auto kernel = mlp_short(M, K, H) ? gelu_mlp_short_f32_kernel : gelu_mlp_f32_kernel;
+    kernel<<<grid, MLP_THREADS, lds, as_stream(stream)>>>(x, w1, b1, w2, b2, y, part, tickets, M, K,
+                                                          H, N);
     return launch_status("gelu mlp");
 }
 

@@ -22,6 +22,11 @@ from autotuner_runtime import ops  # noqa: E402
     (3, 260, 1028, 260),   # K and N past one batch, 17 chunks with 4 units in the last
     (20, 1024, 2048, 68),  # 32 chunks, four batches of W1
     (8, 20, 100, 321),     # N past 256 and off 4
+    (50, 128, 128, 30),    # the last rows of the small-network form at H = 128
+    (51, 128, 128, 30),    # ... and one past it
+    (8, 56, 288, 259),     # ... past H = 128
+    (9, 56, 288, 259),
+    (3, 164, 8, 5),        # rows too long for it
 ])
 def test_tiny_mlp_tile_edges(M, K, H, N):
     r = rng(6000 + M + K + H + N)
