@@ -1,13 +1,9 @@
 // Rows A2-A4 (+ the A5/A8/A9 region epilogues): affine quantized matmul.
 //
 // y[M, N] = x[M, K] @ dequant(w)^T with w uint32 [N, K*bits/32] (MLX layout),
-// scales/biases T [N, K/gs]. Two kernels, mirroring the library's two regimes
-// (scaffold/stitch.py:74-100, 176-293):
-//
-//  * qmv_kernel (small M, and the generic fallback): 16 lanes per output row,
-//    4 rows per wave; each lane streams 16-byte weight chunks and accumulates
-//    the per-group factored sum s*sum(x*q) + b*sum(x) in fp32
-//    (lower.py:1179-1233); a 16-lane xor-shuffle tree reduces the row.
+// scales/biases T [N, K/gs]. Two regimes, the library's (scaffold/stitch.py:74-100,
+// 176-293): up to 8 tokens, and shapes the one below does not take, the GEMV
+// kernels of mi_gemv.hip (gemv_launch); else
 //
 //  * qmm_mfma_kernel (M > 8, bf16/fp16): 32x32x16 MFMA with the weight tile
 //    as the A operand (rows = output features) and x^T as B (columns =
@@ -1191,7 +1187,10 @@ int launch_mfma_mixed3(QParams p, int nb, int cus, hipStream_t st) {
 // at K = 2560, to N 1024 / 2048 / 2560 / 6144 by K 2048 to 9728 and the duals
 // N 8192 and 9728 at 129, 200, 256, 320, 384 and 501 tokens, 4 and 8 bits
 // (features x tokens): 32x32 58 + 37, 32x64 71 + 51, 32x128 98 + 88, 64x64
-// 94 + 82, 64x128 134 + 125. Before, 32x64 below 512 tokens or 32x32 past a
+// 94 + 82, 64x128 134 + 125 (8 bits, one part: 121 + 112; with 4 bits' figures
+// 64x64 and 64x128 tied where the larger is the faster: 11528 x 3840 at 224 tokens
+// 42.6 against 49.2, 5380 x 5376 at 542 61 / 76). Groups 32 and 128, fp16 and K from
+// 512 follow the same figures (over random shapes 1.1x before's choice). Before, 32x64 below 512 tokens or 32x32 past a
 // K of about 9000, 64x128 from 512, and two thresholds on the width between.
 // 4 bits, 501 tokens: 6144 x 2560 33.6 -> 26.7 us, 2560 x 4096 24.7 -> 19.7,
 // 2560 x 9728 63.8 -> 40.3, 2048 x 8192 44.7 -> 26.5; dual 9728 x 2560 at 384
@@ -1248,7 +1247,8 @@ int launch_mfma(const QParams &p, hipStream_t st) {
             }
             if (al2 && (P == 1 || nt * ceil_div(p.M, 64) >= 128)) {
                 offer(T22, mfma_lds_bytes<T, BITS, 2, 2>(p, wk), 3 - P, 2, 94, 82);
-                offer(T24, mfma_lds_bytes<T, BITS, 2, 4>(p, wk), 3 - P, 4, 134, 125);
+                constexpr int less = BITS == 8 && P == 1 ? 13 : 0;
+                offer(T24, mfma_lds_bytes<T, BITS, 2, 4>(p, wk), 3 - P, 4, 134 - less, 125 - less);
             }
             if constexpr (P == 1) {
                 if (best == T11) return launch_mfma_cfg<T, BITS, 1, 1, EPI>(p, wk, st);

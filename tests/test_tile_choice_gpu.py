@@ -57,3 +57,28 @@ def test_dual_tile_choice(M, N, K):
     y1, y2 = ops.qmm_dual(x, *one, *two)
     assert torch.equal(y1, ops.quantized_matmul(x, *one))
     assert torch.equal(y2, ops.quantized_matmul(x, *two))
+
+
+# (M, parts): grids whose cheapest tile is, on 256 CUs, 32 x 32, 32 x 64, 64 x 64,
+# 64 x 128 and, for parts that are no multiples of 64 features, 32 x 128; a ragged
+# last token tile each
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,Ns", [(131, (256, 64, 128)), (261, (512, 256, 256)),
+                                  (301, (1024, 512, 512)), (1025, (4096, 1024, 1024)),
+                                  (1025, (4096, 1024, 1056))])
+def test_grouped_tile_choice(M, Ns, bits):
+    """Each part equals its own launch, which has another grid and tile."""
+    print(f"\ngrouped tile choice M={M} parts={Ns} {bits}-bit", flush=True)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(M + sum(Ns) + bits)
+    K = 512
+    x = torch.randn(M, K, generator=gen, device="cuda").bfloat16()
+    parts = [random_quantized(n, K, gen, "cuda", 64, bits, torch.bfloat16) for n in Ns]
+    for y, p in zip(ops.qmm_grouped3(x, parts, 64, bits), parts):
+        assert torch.equal(y, ops.quantized_matmul(x, *p, bits=bits))
+        W = ops.dequantize(*p, bits=bits).double()
+        want = x.double() @ W.t().contiguous()
+        # half an ulp of the value and the fp32 sums' error, as above
+        size = x.double().abs() @ W.abs().t().contiguous()
+        assert bool(((y.double() - want).abs()
+                     <= 2.0 ** -8 * want.abs() + K * 2.0 ** -24 * size).all())
