@@ -39,7 +39,7 @@ FLAGS = [
 # Per-source device flags. mi_attn.hip: MFMA results in arch VGPRs. By
 # default the compiler kept the attention accumulators in AGPRs and copied
 # them through VGPRs for every tile's softmax rescale and stream merge
-# (272 v_accvgpr_read/write in the 64-wide shared kernel, about 40 % of its
+# (272 v_accvgpr_read/write in the 64-wide form, about 40 % of its
 # loop's VALU), which also cost occupancy. Same instructions otherwise, same
 # results.
 SOURCE_FLAGS = {"mi_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}

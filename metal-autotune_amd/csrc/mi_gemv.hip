@@ -204,7 +204,7 @@ constexpr bool qmv_dot2_wide_ok(int epi) { return epi_parts(epi) == 1 && epi != 
 template <typename T, int MR, int EPI, bool PF = false, bool WIDE = false, int LPR = 16>
 __global__ __launch_bounds__(WIDE ? 1024 : 256) void qmv_dot2_kernel(QParams p) {
     static_assert(!WIDE || qmv_dot2_wide_ok(EPI), "wide workgroups: single output");
-    static_assert(LPR == 16 || (LPR == 64 && qmv_dot2_wide_ok(EPI)), "a row a wave: single output");
+    static_assert(LPR == 16 || LPR == 64, "4 rows or one a wave");
     static_assert(!PF || MR == 1, "PF: one token");
     static_assert(!PF || !WIDE || LPR == 64, "PF in wide workgroups: a row a wave");
     constexpr int RPW = 64 / LPR;  // rows a wave
@@ -753,8 +753,11 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
     const int64_t gy = ceil_div(p.M, mr);
     const bool pf = epi_parts(EPI) == 1 && mr == 1 && ceil_div(p.Nout, 16) * gy <= 1024 &&
                     p.K / 8 <= 512;
-    // A row a wave (LPR 64) for single-output launches over long rows (K >
-    // 4096, more than 8 chunks a lane at 16 lanes a row). Waves per workgroup
+    // A row a wave (LPR 64) over long rows (K > 4096, more than 8 chunks a lane
+    // at 16 lanes a row), whatever the epilogue: it is another order of sums. The
+    // dual gains to 4096 features (1 token, x 8192 15.1 -> 8.6 us) and pays past
+    // them (14336 x 5120 17.7 -> 20.0, 2 tokens 20 -> 28).
+    // Waves per workgroup
     // without PF: as many as spread the rows evenly over the CUs in one round
     // of workgroups (N = 9728 at 4 rows a wave: 10 waves, 244 workgroups, at
     // most 40 rows a CU, where 16-row workgroups put 48 on some CUs and 32 on
@@ -763,7 +766,7 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
     // epilogue, whose workgroups each lie inside one part, and for the
     // several-output ones.
     constexpr bool wide_ok = qmv_dot2_wide_ok(EPI);
-    const bool row_wave = wide_ok && !pf && p.K / 32 > 128;
+    const bool row_wave = p.K / 32 > 128;  // (pf: K <= 4096)
     const int rpw = row_wave ? 1 : 4;
     int waves = 4;
     if constexpr (wide_ok) {
@@ -782,19 +785,19 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
             qmv_dot2_kernel<T, 2, EPI><<<grid, bs, lds, st>>>(p);
         else
             qmv_dot2_kernel<T, 4, EPI><<<grid, bs, lds, st>>>(p);
-    } else if constexpr (wide_ok) {
+    } else if (waves == 4) {
         // a row a wave takes PF too at M = 1 while x fits two chunks a thread
-        // (Qwen3's down_proj at decode, 10-wave workgroups: 6.7 -> 5.6 us)
+        // (Qwen3's down_proj at decode, 10-wave workgroups: 6.7 -> 5.6 us), single
+        // output
+        if (mr == 1 && wide_ok && p.K / 8 <= 2 * bs)
+            qmv_dot2_kernel<T, 1, EPI, wide_ok, false, 64><<<grid, bs, lds, st>>>(p);
+        else if (mr == 1)
+            qmv_dot2_kernel<T, 1, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
+        else
+            qmv_dot2_kernel<T, 2, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
+    } else if constexpr (wide_ok) {
         if (row_wave && mr == 1 && p.K / 8 <= 2 * bs) {
-            if (waves == 4)
-                qmv_dot2_kernel<T, 1, EPI, true, false, 64><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 1, EPI, true, true, 64><<<grid, bs, lds, st>>>(p);
-        } else if (row_wave && waves == 4) {
-            if (mr == 1)
-                qmv_dot2_kernel<T, 1, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 2, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
+            qmv_dot2_kernel<T, 1, EPI, true, true, 64><<<grid, bs, lds, st>>>(p);
         } else if (row_wave) {
             if (mr == 1)
                 qmv_dot2_kernel<T, 1, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);

@@ -100,6 +100,23 @@ def test_few_token_epilogues_agree_at_long_rows(K, gs, bits, M):
     assert float((t.double() - want).abs().max()) <= 1e-2 * float(want.abs().max())
 
 
+@pytest.mark.parametrize("M,K", [(1, 4096), (1, 4160), (2, 5120), (2, 9728)])
+def test_decode_epilogues_agree_at_long_rows(M, K):
+    """One or two tokens at 4 bits: a row a wave past K = 4096, in every epilogue."""
+    D = 1024
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(K + M)
+    xd = torch.randn((1, M, K), generator=gen, device="cuda").half()
+    w, w2 = (random_quantized(3 * D, K, gen, "cuda", 64, 4, torch.float16) for _ in range(2))
+    t, u = (ops.quantized_matmul(xd, *a) for a in (w, w2))
+    y1, u1 = ops.qmm_dual(xd, *w, *w2)
+    assert torch.equal(y1, t) and torch.equal(u1, u)
+    c, bx = ops.qmm_split_gate(xd, *w)
+    assert torch.equal(c, t[..., D:2 * D]) and torch.equal(bx, t[..., :D] * t[..., 2 * D:])
+    for y, a in zip(ops.qmm_grouped3(xd, (w, w2, w)), (t, u, t)):
+        assert torch.equal(y, a)
+
+
 @pytest.mark.parametrize("N,K,bits", [(2033, 320, 4), (2048, 320, 4), (2033, 576, 8)])
 def test_few_token_epilogues_agree_at_unaligned_scales(N, K, bits):
     """One weight of a pair is a view whose scales and biases lie off a 16-byte

@@ -590,10 +590,10 @@ def test_qmm_grouped3_mixed_tiles_qwen3_shape(M):
 
 @pytest.mark.parametrize("Ns,bits", [((256, 64, 128), 4), ((256, 96, 64), 4), ((128, 64, 64), 8)])
 def test_qmm_grouped3_large_m_tiles(Ns, bits):
-    """From M = 512 the grouped launch takes 64-feature tiles when every part
-    is a multiple of 64, else 32-feature tiles: both bit for bit equal to the
-    three separate launches (which take their own tiles), and within the
-    oracle's tolerance on the first rows."""
+    """At M = 520 (the interleaved K split) the grouped launch is bit for bit
+    equal to the three separate launches (which take their own tiles), and
+    within the oracle's tolerance on the first rows. (These narrow parts take
+    32-feature tiles; the wider ones are in test_tile_choice_gpu.py.)"""
     r = rng(760 + sum(Ns) + bits)
     M, K = 520, 512
     x = oracle.round_to(r.normal(0, 1, (1, M, K)), "bfloat16")
@@ -759,14 +759,14 @@ def test_sdpa(H, HK, Lq, Lk, D, causal):
                                              (32, 8, 512, 128, False), (32, 8, 544, 64, False)])
 def test_sdpa_shared_and_split_kernels_agree(H, HK, L, D, causal):
     """A row's attention is the same bits whichever kernel computes it. The
-    L-row call runs the shared-K/V kernel (a grid of at least 128
-    workgroups, causal q blocks paired long with short); a call on its last
-    32 query rows, and a decode call on its last row, run the key-split
-    kernel (smaller grids) over the same keys. Causal at head dim 64, the q
-    blocks with 1, 2, 3, 5 and 8 key tiles (fewer streams than four, streams
-    of unequal length) are also checked against split-kernel calls over
-    their own visible keys. L = 544 (17 tiles, no mask, an odd block count:
-    no pairing) gives stream 0 one tile more than the others."""
+    L-row call runs the kernel whose units share staged key tiles (a grid of at
+    least 192 workgroups of two) or, smaller, a unit a workgroup; a call on its
+    last 32 query rows, and a decode call on its last row (the heads' rows as
+    one tile's columns), run the latter's forms over the same keys. Causal at
+    head dim 64, the q blocks with 1, 2, 3, 5 and 8 key tiles (fewer streams
+    than four, streams of unequal length) are also checked against calls over
+    their own visible keys. L = 544 (17 tiles, no mask) gives stream 0 one tile
+    more than the others."""
     r = rng(1050 + L + D)
     q = to_torch(oracle.round_to(r.normal(0, 1, (1, H, L, D)), "bfloat16"), "bfloat16")
     k = to_torch(oracle.round_to(r.normal(0, 1, (1, HK, L, D)), "bfloat16"), "bfloat16")
