@@ -815,17 +815,23 @@ int launch_decode(const AttnArgs &a, float *ws, hipStream_t st) {
     return launch_status("sdpa (decode)");
 }
 
-// Two units (q heads' 32-row blocks) share each staged K/V tile while that
-// leaves a workgroup for most CUs (half the K/V traffic, two waves a SIMD);
-// else one unit a workgroup, of which a CU holds two and whose waves wait for
-// no barrier (64 tokens 5.05 us against 6.2 for one unit through the shared
-// stages, 16 behind 4080 26.6 against 35). Same results.
+// Two units (q heads' 32-row blocks) share each staged K/V tile where that leaves
+// a workgroup for most CUs and the rows are long (half the K/V traffic, two waves a
+// SIMD); else one unit a workgroup, of which a CU holds two and whose waves wait
+// for no barrier (64 tokens 5.05 us against 6.2 for one unit through the shared
+// stages, 16 behind 4080 26.6 against 35). Short rows fill few of the stages: 205
+// tokens, 64/8 heads of 64 5.2 / 6.4; 265 tokens, 64/8 of 128 10.1 / 14.4; 16 x 289
+// tokens 114 / 150. Past 256 keys only while K and V of all heads (a unit reads
+// its own copy) stay in the caches: 8 x 436 tokens, 64/32 heads of 128 (57 MB) 226
+// / 161. Same results.
 template <typename T, int D>
 int launch_attn_d(const AttnArgs &a, float *ws, hipStream_t st) {
     if (a.Lq <= DEC_MAX_LQ) return launch_decode<T, D>(a, ws, st);
     const int64_t rep = a.H / a.HK, units = rep * ceil_div(a.Lq, 32), nbk = a.B * a.HK;
     const int64_t nub = ceil_div(units, 2);
-    if (nbk * nub >= 192)
+    const bool short_rows =
+        a.Lk <= 256 || (a.Lk <= 640 && nbk * a.Lk * D * 4 <= ((int64_t)40 << 20));
+    if (nbk * nub >= 192 && !short_rows)
         attn_prefill_kernel<T, D, 2><<<(unsigned)(nbk * nub), 512, 0, st>>>(
             (const T *)a.q, (const T *)a.k, (const T *)a.v, (T *)a.out, a.H, a.Lq, a.Lk, a.cap,
             a.scale, a.flip, a.causal, a.out_layout, make_div(nbk, nbk * nub),

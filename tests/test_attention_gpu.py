@@ -34,9 +34,13 @@ def _close(got, want, tol=1e-2):
     (1, 3, 1, 1, 16500, 64, True, 1, "bfloat16"),     # one kv head: 129 splits
     (1, 8, 2, 9, 9, 64, True, 1, "bfloat16"),         # first size past decode
     (1, 8, 2, 33, 1100, 128, True, 1, "float16"),     # a second row block of one row
-    (3, 15, 3, 417, 417, 64, True, 1, "bfloat16"),    # shared tiles, odd unit count, q heads 5 a group
-    (1, 32, 8, 400, 431, 128, True, 1, "bfloat16"),   # shared tiles, ragged chunk behind a prefix
-    (1, 32, 8, 384, 384, 64, False, 1, "float16"),    # shared tiles, no mask
+    (3, 15, 3, 417, 417, 64, True, 1, "bfloat16"),    # a unit a workgroup, q heads 5 a group
+    (1, 32, 8, 400, 431, 128, True, 1, "bfloat16"),   # ... ragged chunk behind a prefix
+    (1, 32, 8, 384, 384, 64, False, 1, "float16"),    # ... no mask
+    (1, 32, 8, 400, 731, 128, True, 1, "bfloat16"),   # past 640 keys: shared tiles
+    (1, 32, 8, 384, 644, 64, False, 1, "float16"),
+    (2, 15, 3, 641, 641, 64, True, 1, "bfloat16"),    # ... an odd unit count, q heads 5 a group
+    (1, 32, 8, 390, 741, 128, True, -1, "bfloat16"),
     (1, 8, 2, 1, 70, 128, True, -1, "bfloat16"),      # a negative scale
     (1, 32, 8, 390, 390, 128, True, -1, "bfloat16"),
     (1, 8, 2, 40, 70, 64, True, 0, "bfloat16"),       # scale 0: the mean of the visible values
@@ -88,7 +92,7 @@ def test_sdpa_without_a_workspace(Lq, Lk):
     (8, 2, 1, 128, 128),      # decode
     (8, 2, 2, 2048, 64),      # ... split
     (8, 2, 32, 160, 64),      # few query rows
-    (32, 8, 400, 512, 128),   # shared tiles
+    (32, 8, 400, 672, 128),   # shared tiles
 ])
 @pytest.mark.parametrize("gap", [25.0, 150.0])
 def test_sdpa_one_large_score(H, HK, Lq, Lk, D, gap, dtype):
@@ -114,7 +118,7 @@ def test_sdpa_one_large_score(H, HK, Lq, Lk, D, gap, dtype):
     (8, 2, 1, 992, 128),      # decode
     (8, 2, 2, 2048, 64),      # ... split
     (8, 2, 32, 160, 64),      # few query rows
-    (32, 8, 400, 512, 128),   # shared tiles
+    (32, 8, 400, 672, 128),   # shared tiles
 ])
 def test_sdpa_row_sum_adds_unrounded_weights(H, HK, Lq, Lk, D, dtype):
     """In every tile of 32 keys one has weight 1 and value 1, the others weight p
@@ -137,7 +141,7 @@ def test_sdpa_row_sum_adds_unrounded_weights(H, HK, Lq, Lk, D, dtype):
     assert bool((o == want.cuda()).all()), (float(o.min()), float(o.max()), float(want))
 
 
-@pytest.mark.parametrize("Lq,Lk", [(1, 40), (2, 1500), (40, 40), (400, 400)])
+@pytest.mark.parametrize("Lq,Lk", [(1, 40), (2, 1500), (40, 40), (400, 700)])
 def test_sdpa_scale_of_nan(Lq, Lk):
     q, k = torch.ones((1, 32, Lq, 64), device="cuda").bfloat16(), torch.ones(
         (1, 8, Lk, 64), device="cuda").bfloat16()

@@ -737,7 +737,8 @@ def test_norm_rope_qkv_equals_three_calls(L, offset, strided):
                                                  (8, 8, 40, 70, 64, True),
                                                  (6, 2, 33, 33, 128, False),
                                                  (12, 4, 5, 130, 128, True),
-                                                 (32, 8, 512, 512, 64, True),      # shared-K/V kernel
+                                                 (32, 8, 512, 512, 64, True),      # a unit a workgroup
+                                                 (32, 8, 672, 672, 64, True),      # shared key tiles
                                                  (16, 2, 1000, 1030, 128, True)])  # shared, 2 quads
 def test_sdpa(H, HK, Lq, Lk, D, causal):
     r = rng(1000 + Lq + Lk + D)
@@ -756,11 +757,12 @@ def test_sdpa(H, HK, Lq, Lk, D, causal):
 
 
 @pytest.mark.parametrize("H,HK,L,D,causal", [(32, 8, 512, 64, True), (16, 2, 1024, 128, True),
-                                             (32, 8, 512, 128, False), (32, 8, 544, 64, False)])
+                                             (32, 8, 512, 128, False), (32, 8, 544, 64, False),
+                                             (32, 8, 672, 64, True), (32, 8, 704, 128, False)])
 def test_sdpa_shared_and_split_kernels_agree(H, HK, L, D, causal):
     """A row's attention is the same bits whichever kernel computes it. The
-    L-row call runs the kernel whose units share staged key tiles (a grid of at
-    least 192 workgroups of two) or, smaller, a unit a workgroup; a call on its
+    L-row call runs the kernel whose units share staged key tiles (past 640 keys,
+    a grid of at least 192 workgroups of two), else a unit a workgroup; a call on its
     last 32 query rows, and a decode call on its last row (the heads' rows as
     one tile's columns), run the latter's forms over the same keys. Causal at
     head dim 64, the q blocks with 1, 2, 3, 5 and 8 key tiles (fewer streams
