@@ -43,13 +43,13 @@
 // calls (at most DEC_MAX_LQ rows over more than DEC_SPLIT_MIN_LK keys, with a
 // workspace), a short last chunk among them, agree within rounding.
 //
-// What bounds it: at long prompts the softmax VALU, about 65 instructions and
-// 16 v_exp (a quarter-rate unit) for the 16 MFMAs of a tile at D = 128, 8 at D =
-// 64, and its waves' turns (two a SIMD at D = 128); for decode one memory round
+// What bounds it: at long prompts the softmax VALU, some 60 instructions and 16
+// v_exp (a quarter-rate unit) for the 16 MFMAs of a tile at D = 128, 8 at D = 64
+// (143 VALU a tile counted with everything in), and its waves' turns (two a SIMD at D = 128); for decode one memory round
 // trip and the launches. Measured on MI355X in a graph, 32 q / 8 kv heads (in
 // brackets: a form that masked and rescaled every score with 360 VALU a tile,
 // staged tiles through registers, and ran decode on one workgroup per q head):
-// 2048 tokens D = 128 60 us (85), D = 64 30 (60); 501 behind 777, D = 128, 19
+// 2048 tokens D = 128 61 us (85), D = 64 30 (60); 501 behind 777, D = 128, 19
 // (54); 128 tokens 5.6 (6.5); decode over 129 keys 5.2 (7.6), 1001 9.6 (18.8),
 // 8191 11.5 us, 2.9 TB/s of K and V (115).
 #include <math.h>
