@@ -475,17 +475,22 @@ template <int PER, int N> __device__ __forceinline__ void wait_units(int n) {
 
 // Dynamic LDS: x rows (a 16-byte pad a row, so the rows' reads of one chunk
 // spread over the banks), the scale and bias rows; the partial sums reuse it.
+// spread: beside them (the waves finish runs while others still read).
 struct QmsLds {
-    int pitch, sb, total;  // bytes: of an x row; of one scale or bias array
+    int pitch, sb, red, total;  // bytes: of an x row; of one scale or bias array
 };
-__host__ __device__ inline QmsLds qms_lds(int rows, int64_t K, int64_t G, int parts, int waves) {
+__host__ __device__ inline QmsLds qms_lds(int rows, int64_t K, int64_t G, int parts, int runs,
+                                          bool spread = false) {
     const int pitch = (int)(2 * K) + 16, sb = (int)(16 * G * 2);
-    const int stage = rows * pitch + 2 * parts * sb, red = waves * parts * 1024;
-    return {pitch, sb, stage > red ? stage : red};
+    const int stage = rows * pitch + 2 * parts * sb, red = runs * parts * 1024;
+    if (spread) return {pitch, sb, stage, stage + red};
+    return {pitch, sb, 0, stage > red ? stage : red};
 }
-// Waves of a workgroup, a function of K alone: about 8 groups of 64 a wave at
-// the projection widths.
-inline int qms_waves(int64_t K) { return K > 4096 ? 16 : 8; }
+// Runs of K, whose sums are added in order: a function of K alone, about 8 groups
+// of 64 a run at the projection widths. A wave takes one; or two in turn where 16
+// waves, of which a CU holds one workgroup, would leave the last round of
+// workgroups nearly empty (see launch_qms).
+inline int qms_runs(int64_t K) { return K > 4096 ? 16 : 8; }
 
 // bind() of an epilogue known at run time (EPI_GROUP3 among the single-part ones).
 template <int P> __device__ __forceinline__ Bound bind_of(const QParams &p, int epi, int64_t &nb) {
@@ -508,8 +513,8 @@ template <int P> __device__ __forceinline__ Bound bind_of(const QParams &p, int 
 }
 
 template <typename T, int BITS, int P, int GSL, bool PAIR>
-__global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, int nw, int run,
-                                                   int longer, int sb_dma) {
+__global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, int nw, int runs,
+                                                   int run, int longer, int sb_dma) {
 #if defined(__HIP_DEVICE_COMPILE__)
     typedef QmsShape<BITS, P, GSL, PAIR> Sh;
     typedef __attribute__((address_space(3))) void *lds_ptr;
@@ -524,7 +529,7 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
     const int rows = (int)(p.M - m0 < mr ? p.M - m0 : mr);
     const int64_t K = p.K;
     const int G = (int)(K >> GSL);
-    const QmsLds L = qms_lds(rows, K, G, P, nw);
+    const QmsLds L = qms_lds(rows, K, G, P, runs, runs > nw);
     char *sbl = qlds + rows * L.pitch;  // [part][scale, bias][16][G]
 
     // x rows, then the scale and bias rows, 16 bytes a lane; the instructions
@@ -570,10 +575,11 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
     }
     __builtin_amdgcn_sched_barrier(0);
 
-    // this wave's units (run + 1 for the first `longer` waves, run for the rest),
-    // and the first GB of them (rows past N read a clamped, valid address)
-    const int u0 = wave * run + (wave < longer ? wave : longer);
-    const int u1 = u0 + run + (wave < longer ? 1 : 0);
+    // this wave's (first) run: its units (run + 1 for the first `longer` runs, run
+    // for the rest), and the first GB of them (rows past N read a clamped, valid
+    // address)
+    int u0 = wave * run + (wave < longer ? wave : longer);
+    int u1 = u0 + run + (wave < longer ? 1 : 0);
     const int64_t n = nb + nl;
     const int64_t nrow = n < bd.Nout ? n : bd.Nout - 1;
     const uint32_t *wr[P];
@@ -690,23 +696,33 @@ __global__ __launch_bounds__(1024) void qms_kernel(QParams p, int epi, int mr, i
         }
     }
     };
-    body(xrow, srow);
-
-    // the waves' sums, in wave order: token 4 kb + e of feature nl is element e
-    // of lane (kb, nl); wave e < 4 adds and stores element e
-    __syncthreads();
-    float *red = (float *)qlds;
+    // the runs' sums, in order: token 4 kb + e of feature nl is element e of lane
+    // (kb, nl); wave e < 4 adds and stores element e
+    float *red = (float *)(qlds + L.red);
+    for (int vw = wave;;) {  // (wave-uniform)
+        body(xrow, srow);
+        if (runs == nw) __syncthreads();  // (the sums take the staged rows' place)
 #pragma unroll
-    for (int q = 0; q < P; ++q)
-        *(float4 *)(red + ((wave * P + q) * 64 + lane) * 4) =
-            make_float4(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
+        for (int q = 0; q < P; ++q) {
+            *(float4 *)(red + ((vw * P + q) * 64 + lane) * 4) =
+                make_float4(acc[q][0], acc[q][1], acc[q][2], acc[q][3]);
+            acc[q] = zero;
+        }
+        vw += nw;
+        if (vw >= runs) break;
+        u0 = vw * run + (vw < longer ? vw : longer);
+        u1 = u0 + run + (vw < longer ? 1 : 0);
+#pragma unroll
+        for (int i = 0; i < GB; ++i)
+            if (i < u1 - u0) load(i, u0 + i);
+    }
     __syncthreads();
     if (wave >= 4) return;
     float v[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
         v[q] = red[(q * 64 + lane) * 4 + wave];
-        for (int s = 1; s < nw; ++s) v[q] += red[((s * P + q) * 64 + lane) * 4 + wave];
+        for (int s = 1; s < runs; ++s) v[q] += red[((s * P + q) * 64 + lane) * 4 + wave];
     }
     const int t = 4 * kb + wave;
     if (t >= rows || n >= bd.Nout) return;
@@ -821,12 +837,12 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
 // adds in its order) or none does.
 inline bool qms_takes(int64_t M, int64_t K, int gs_log2) {
     return M <= QMV_MR && K < ((int64_t)1 << 24) &&
-           qms_lds(1, K, K >> gs_log2, 3, qms_waves(K)).total <= LDS_PER_CU;
+           qms_lds(1, K, K >> gs_log2, 3, qms_runs(K)).total <= LDS_PER_CU;
 }
 // Token rows per workgroup: all of them, halved while x does not fit the LDS.
 inline int qms_rows(const QParams &p, int parts) {
     int mr = (int)p.M;
-    while (mr > 1 && qms_lds(mr, p.K, p.K >> p.gs_log2, parts, qms_waves(p.K)).total > LDS_PER_CU)
+    while (mr > 1 && qms_lds(mr, p.K, p.K >> p.gs_log2, parts, qms_runs(p.K)).total > LDS_PER_CU)
         mr = (mr + 1) / 2;
     return mr;
 }
@@ -843,30 +859,39 @@ inline bool qms_sb_dma(const QParams &p, int epi) {
 }
 
 template <typename T, int BITS, int P, int GSL>
-void launch_qms_gs(const QParams &p, int epi, int mr, dim3 grid, size_t lds, hipStream_t st) {
-    const int G = (int)(p.K >> GSL), nw = qms_waves(p.K), dma = qms_sb_dma(p, epi);
+void launch_qms_gs(const QParams &p, int epi, int mr, int nw, dim3 grid, size_t lds,
+                   hipStream_t st) {
+    const int G = (int)(p.K >> GSL), runs = qms_runs(p.K), dma = qms_sb_dma(p, epi);
     if constexpr (qms_pairs<BITS, GSL>()) {
         if (G % 2 == 0) {
             qms_kernel<T, BITS, P, GSL, true><<<grid, 64 * nw, lds, st>>>(
-                p, epi, mr, nw, G / 2 / nw, G / 2 % nw, dma);
+                p, epi, mr, nw, runs, G / 2 / runs, G / 2 % runs, dma);
             return;
         }
     }
-    qms_kernel<T, BITS, P, GSL, false><<<grid, 64 * nw, lds, st>>>(p, epi, mr, nw, G / nw, G % nw,
-                                                                   dma);
+    qms_kernel<T, BITS, P, GSL, false><<<grid, 64 * nw, lds, st>>>(p, epi, mr, nw, runs, G / runs,
+                                                                   G % runs, dma);
 }
 
 template <typename T, int BITS, int P>
 int launch_qms(const QParams &p, int epi, int mr, hipStream_t st) {
     const dim3 grid((unsigned)ceil_div(p.Nout, 16), (unsigned)ceil_div(p.M, mr));
-    const int nw = qms_waves(p.K);
-    const size_t lds = (size_t)qms_lds(mr, p.K, p.K >> p.gs_log2, P, nw).total;
+    const int64_t G = p.K >> p.gs_log2;
+    int nw = qms_runs(p.K);
+    size_t lds = (size_t)qms_lds(mr, p.K, G, P, nw).total;
+    // Eight waves of two runs past one 16-wave workgroup a CU, while two such
+    // workgroups fit its LDS. Same sums. 8-bit, one token, 12000 x 8192 29.8 -> 21.4
+    // us, 5040 x 5120 10.5 -> 8.7; 4-bit, 3 tokens, 12000 x 5120 14.3 -> 9.5.
+    if (nw == 16 && (int64_t)grid.x * grid.y > device_cus()) {
+        const int spread = qms_lds(mr, p.K, G, P, nw, true).total;
+        if (2 * spread <= LDS_PER_CU) nw = 8, lds = (size_t)spread;
+    }
     if (p.gs_log2 == 5)
-        launch_qms_gs<T, BITS, P, 5>(p, epi, mr, grid, lds, st);
+        launch_qms_gs<T, BITS, P, 5>(p, epi, mr, nw, grid, lds, st);
     else if (p.gs_log2 == 6)
-        launch_qms_gs<T, BITS, P, 6>(p, epi, mr, grid, lds, st);
+        launch_qms_gs<T, BITS, P, 6>(p, epi, mr, nw, grid, lds, st);
     else
-        launch_qms_gs<T, BITS, P, 7>(p, epi, mr, grid, lds, st);
+        launch_qms_gs<T, BITS, P, 7>(p, epi, mr, nw, grid, lds, st);
     return launch_status("quantized matmul (few-token mfma)");
 }
 
@@ -879,7 +904,7 @@ int launch_typed(const QParams &p, int bits, hipStream_t st) {
         // K; the GEMVs / it): 4-bit, 9728 x 2560, M = 2 7.2 / 6.5, M = 4 9.8 / 6.3,
         // M = 8 34 / 6.7; the dual of it M = 2 10.0 / 11.5, M = 4 13.3 / 10.2; 2560 x
         // 9728, M = 2 7.9 / 8.1, M = 4 27 / 7.5, M = 6 50 / 8.0. 8-bit, 2048 x 8192,
-        // M = 1 11.4 / 10.1, M = 6 58 / 11.1, but 5040 x 5120, M = 1 9.0 / 10.6; the
+        // M = 1 11.4 / 10.1, M = 6 58 / 11.1, but 12000 x 5120, M = 1 12.4 / 13.7; the
         // 8192 x 2048 dual M = 1 9.4 / 10.4, M = 2 13.9 / 8.9, M = 6 24 / 9.0; lm_head
         // (151936 x 2560) M = 1 71 / 77, M = 8 445 / 92.
         // Short rows stay with the GEMVs, which have less to set up: 8-bit M = 2,
