@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void qmv_kernel(QParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Decode GEMV (M <= 2, up to K = 512 M <= 4; 4-bit, bf16/fp16): the nibbles never go through a
+// Decode GEMV (one token; two up to K = 4096, four up to K = 512; 4-bit, bf16/fp16): the nibbles never go through a
 // float conversion. (w >> 4j) & 0x000F000F | MAGIC packs nibbles j and j+4 of a
 // word as the two 16-bit floats MAG + q exactly (bf16: 0x4300 = 128, ulp 1 up
 // to 256; fp16: 0x6400 = 1024, ulp 1), so one v_and_or makes a pair and
@@ -772,7 +772,7 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
     // A row a wave (LPR 64) over long rows (K > 4096, more than 8 chunks a lane
     // at 16 lanes a row), whatever the epilogue: it is another order of sums. The
     // dual gains to 4096 features (1 token, x 8192 15.1 -> 8.6 us) and pays past
-    // them (14336 x 5120 17.7 -> 20.0, 2 tokens 20 -> 28).
+    // them (14336 x 5120 17.7 -> 20.0).
     // Waves per workgroup
     // without PF: as many as spread the rows evenly over the CUs in one round
     // of workgroups (N = 9728 at 4 rows a wave: 10 waves, 244 workgroups, at
@@ -802,31 +802,24 @@ int launch_qmv_dot2(const QParams &p, int mr, hipStream_t st) {
         else
             qmv_dot2_kernel<T, 4, EPI><<<grid, bs, lds, st>>>(p);
     } else if (waves == 4) {
-        // a row a wave takes PF too at M = 1 while x fits two chunks a thread
-        // (Qwen3's down_proj at decode, 10-wave workgroups: 6.7 -> 5.6 us), single
-        // output
-        if (mr == 1 && wide_ok && p.K / 8 <= 2 * bs)
+        // a row a wave (one token: see launch_typed) takes PF too while x fits two
+        // chunks a thread (Qwen3's down_proj at decode, 10-wave workgroups: 6.7 ->
+        // 5.6 us), single output
+        if (wide_ok && p.K / 8 <= 2 * bs)
             qmv_dot2_kernel<T, 1, EPI, wide_ok, false, 64><<<grid, bs, lds, st>>>(p);
-        else if (mr == 1)
-            qmv_dot2_kernel<T, 1, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
         else
-            qmv_dot2_kernel<T, 2, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
+            qmv_dot2_kernel<T, 1, EPI, false, false, 64><<<grid, bs, lds, st>>>(p);
     } else if constexpr (wide_ok) {
-        if (row_wave && mr == 1 && p.K / 8 <= 2 * bs) {
+        if (row_wave && p.K / 8 <= 2 * bs)
             qmv_dot2_kernel<T, 1, EPI, true, true, 64><<<grid, bs, lds, st>>>(p);
-        } else if (row_wave) {
-            if (mr == 1)
-                qmv_dot2_kernel<T, 1, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 2, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
-        } else {
-            if (mr == 1)
-                qmv_dot2_kernel<T, 1, EPI, false, true><<<grid, bs, lds, st>>>(p);
-            else if (mr == 2)
-                qmv_dot2_kernel<T, 2, EPI, false, true><<<grid, bs, lds, st>>>(p);
-            else
-                qmv_dot2_kernel<T, 4, EPI, false, true><<<grid, bs, lds, st>>>(p);
-        }
+        else if (row_wave)
+            qmv_dot2_kernel<T, 1, EPI, false, true, 64><<<grid, bs, lds, st>>>(p);
+        else if (mr == 1)
+            qmv_dot2_kernel<T, 1, EPI, false, true><<<grid, bs, lds, st>>>(p);
+        else if (mr == 2)
+            qmv_dot2_kernel<T, 2, EPI, false, true><<<grid, bs, lds, st>>>(p);
+        else
+            qmv_dot2_kernel<T, 4, EPI, false, true><<<grid, bs, lds, st>>>(p);
     }
     return launch_status("quantized matmul (dot2 qmv)");
 }
@@ -899,11 +892,11 @@ template <typename T, int EPI>
 int launch_typed(const QParams &p, int bits, hipStream_t st) {
     if constexpr (sizeof(T) == 2) {
         // The few-token kernel from three tokens (4-bit) or two (8-bit), and for
-        // 8-bit rows past K = 4096 at one; a function of M, K, the width and the
+        // rows past K = 4096 from two or one; a function of M, K, the width and the
         // group size, so every epilogue at one shape adds alike. Measured (us, N x
         // K; the GEMVs / it): 4-bit, 9728 x 2560, M = 2 7.2 / 6.5, M = 4 9.8 / 6.3,
         // M = 8 34 / 6.7; the dual of it M = 2 10.0 / 11.5, M = 4 13.3 / 10.2; 2560 x
-        // 9728, M = 2 7.9 / 8.1, M = 4 27 / 7.5, M = 6 50 / 8.0. 8-bit, 2048 x 8192,
+        // 9728, M = 2 7.9 / 7.1, M = 4 27 / 7.5, M = 6 50 / 8.0. 8-bit, 2048 x 8192,
         // M = 1 11.4 / 10.1, M = 6 58 / 11.1, but 12000 x 5120, M = 1 12.4 / 13.7; the
         // 8192 x 2048 dual M = 1 9.4 / 10.4, M = 2 13.9 / 8.9, M = 6 24 / 9.0; lm_head
         // (151936 x 2560) M = 1 71 / 77, M = 8 445 / 92.
@@ -912,7 +905,7 @@ int launch_typed(const QParams &p, int bits, hipStream_t st) {
         // 4.2 / 3.4; 4-bit M = 3, 2048 x 512 3.1 / 3.3, x 768 3.7 / 3.6.
         constexpr int P = epi_parts(EPI);
         const int64_t M = p.M;
-        const bool few = bits == 4 ? M > 4 || (M > 2 && p.K > 512)
+        const bool few = bits == 4 ? M > 4 || (M > 1 && p.K > (M > 2 ? 512 : 4096))
                                    : p.K > (M == 1 ? 4096 : M == 2 ? 768 : 256);
         if (few && qms_takes(M, p.K, p.gs_log2)) {
             const int rows = qms_rows(p, P);
@@ -920,7 +913,8 @@ int launch_typed(const QParams &p, int bits, hipStream_t st) {
                              : launch_qms<T, 8, P>(p, EPI, rows, st);
         }
         const int mr = M > 2 ? 4 : (int)M;
-        if (bits == 4 && M <= 4 && qmv_dot2_lds_bytes(mr, p.K) <= 65536)
+        if (bits == 4 && (M == 1 || (M <= 4 && p.K <= 4096)) &&
+            qmv_dot2_lds_bytes(mr, p.K) <= 65536)
             return launch_qmv_dot2<T, EPI>(p, mr, st);
     }
     return bits == 4 ? launch_qmv<T, 4, EPI>(p, st) : launch_qmv<T, 8, EPI>(p, st);
